@@ -12,8 +12,9 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libcardiacgpu.so")
-SOURCES = ["model_fp64.hip", "model_fp32.hip", "tissue_implicit.hip", "ldu_solver.hip",
-           "adjoint.hip", "ecg.hip", "general_mesh.hip", "capi.hip"]
+SOURCES = ["model_fp64_ode.hip", "model_fp32_ode.hip", "model_fp64.hip", "model_fp32.hip",
+           "tissue_implicit.hip", "ldu_solver.hip", "adjoint.hip", "ecg.hip",
+           "general_mesh.hip", "capi.hip"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -30,7 +31,7 @@ FAST_F32 = [
     "-fno-hip-fp32-correctly-rounded-divide-sqrt", "-fno-math-errno", "-freciprocal-math",
     "-fapprox-func", "-fno-signed-zeros", "-fgpu-flush-denormals-to-zero",
 ]
-EXTRA = {"model_fp32.hip": FAST_F32}
+EXTRA = {"model_fp32.hip": FAST_F32, "model_fp32_ode.hip": FAST_F32}
 
 
 def _compile(src):

@@ -287,7 +287,7 @@ void k_cells_protocol(T* __restrict__ st, KParams<T> P, const T* __restrict__ gs
     }
 }
 
-template <class T> struct BatchLaunch {
+template <class T, bool ADAPTIVE> struct BatchLaunch {
     template <class M, int BLOCK, int WPE, int INTEG = 0>
     static hipError_t go(int tissue, void* states, const ModelParams& P, const void* gscale,
                          const BatchArgs& a, hipStream_t s)
@@ -303,36 +303,39 @@ template <class T> struct BatchLaunch {
     static hipError_t variant(int v, int tissue, void* states, const ModelParams& P,
                               const void* gscale, const BatchArgs& a, hipStream_t s)
     {
-        if (a.method == 1) return go<M, 64, 0, 1>(tissue, states, P, gscale, a, s);
-        if (a.method == 2) return go<M, 64, 0, 2>(tissue, states, P, gscale, a, s);
-        switch (v) {
-        case 0: return go<M, 256, 0>(tissue, states, P, gscale, a, s);
-        case 1: return go<M, 64, 0>(tissue, states, P, gscale, a, s);
-        case 2: return go<M, 256, 2>(tissue, states, P, gscale, a, s);
-        case 3: return go<M, 64, 2>(tissue, states, P, gscale, a, s);
-        case 4: return go<M, 256, 3>(tissue, states, P, gscale, a, s);
-        case 5: return go<M, 128, 0>(tissue, states, P, gscale, a, s);
-        default: return hipErrorInvalidValue;
+        if constexpr (ADAPTIVE) {
+            if (a.method == 2) return go<M, 64, 0, 2>(tissue, states, P, gscale, a, s);
+            return go<M, 64, 0, 1>(tissue, states, P, gscale, a, s);
+        } else {
+            switch (v) {
+            case 0: return go<M, 256, 0>(tissue, states, P, gscale, a, s);
+            case 1: return go<M, 64, 0>(tissue, states, P, gscale, a, s);
+            case 2: return go<M, 256, 2>(tissue, states, P, gscale, a, s);
+            case 3: return go<M, 64, 2>(tissue, states, P, gscale, a, s);
+            case 4: return go<M, 256, 3>(tissue, states, P, gscale, a, s);
+            case 5: return go<M, 128, 0>(tissue, states, P, gscale, a, s);
+            default: return hipErrorInvalidValue;
+            }
         }
     }
 };
 
-#define CG_DEFINE_BATCH_ENTRY(T, SFX)                                                      \
+#define CG_DEFINE_BATCH_ENTRY(T, AD, SFX)                                                  \
     hipError_t launch_cells_protocol_##SFX(int model, int tissue, int variant, void* states, \
                                            const ModelParams& P, const void* gscale,       \
                                            const BatchArgs& a, hipStream_t s)              \
     {                                                                                      \
         switch (model) {                                                                   \
-        case MODEL_BO: return BatchLaunch<T>::variant<BuenoOrovio>(variant, tissue, states, P, gscale, a, s); \
-        case MODEL_TNNP: return BatchLaunch<T>::variant<TNNP>(variant, tissue, states, P, gscale, a, s); \
-        case MODEL_ORD: return BatchLaunch<T>::variant<ORd>(variant, tissue, states, P, gscale, a, s); \
-        case MODEL_AP: return BatchLaunch<T>::variant<AlievPanfilov>(variant, tissue, states, P, gscale, a, s); \
-        case MODEL_CRN: return BatchLaunch<T>::variant<Courtemanche>(variant, tissue, states, P, gscale, a, s); \
-        case MODEL_PYS: return BatchLaunch<T>::variant<PerisYague>(variant, tissue, states, P, gscale, a, s); \
-        case MODEL_STW: return BatchLaunch<T>::variant<Stewart>(variant, tissue, states, P, gscale, a, s); \
-        case MODEL_GRD: return BatchLaunch<T>::variant<Grandi>(variant, tissue, states, P, gscale, a, s); \
-        case MODEL_TOR: return BatchLaunch<T>::variant<ToRORd>(variant, tissue, states, P, gscale, a, s); \
-        case MODEL_GAUR: return BatchLaunch<T>::variant<Gaur>(variant, tissue, states, P, gscale, a, s); \
+        case MODEL_BO: return BatchLaunch<T, AD>::variant<BuenoOrovio>(variant, tissue, states, P, gscale, a, s); \
+        case MODEL_TNNP: return BatchLaunch<T, AD>::variant<TNNP>(variant, tissue, states, P, gscale, a, s); \
+        case MODEL_ORD: return BatchLaunch<T, AD>::variant<ORd>(variant, tissue, states, P, gscale, a, s); \
+        case MODEL_AP: return BatchLaunch<T, AD>::variant<AlievPanfilov>(variant, tissue, states, P, gscale, a, s); \
+        case MODEL_CRN: return BatchLaunch<T, AD>::variant<Courtemanche>(variant, tissue, states, P, gscale, a, s); \
+        case MODEL_PYS: return BatchLaunch<T, AD>::variant<PerisYague>(variant, tissue, states, P, gscale, a, s); \
+        case MODEL_STW: return BatchLaunch<T, AD>::variant<Stewart>(variant, tissue, states, P, gscale, a, s); \
+        case MODEL_GRD: return BatchLaunch<T, AD>::variant<Grandi>(variant, tissue, states, P, gscale, a, s); \
+        case MODEL_TOR: return BatchLaunch<T, AD>::variant<ToRORd>(variant, tissue, states, P, gscale, a, s); \
+        case MODEL_GAUR: return BatchLaunch<T, AD>::variant<Gaur>(variant, tissue, states, P, gscale, a, s); \
         default: return hipErrorInvalidValue;                                              \
         }                                                                                  \
     }

@@ -774,11 +774,8 @@ hipError_t batch_launch(cg_ionic* h, double dtm, int64_t s0, int chunk, hipStrea
         a.step = h->d_step;
         a.fail = h->d_fail;
     }
-    return h->prec == CG_FP64
-        ? cg::launch_cells_protocol_fp64(h->model, h->tissue, h->variant, h->d_states, h->P,
-                                         h->d_gscale, a, s)
-        : cg::launch_cells_protocol_fp32(h->model, h->tissue, h->variant, h->d_states, h->P,
-                                         h->d_gscale, a, s);
+    return cg::launch_cells_protocol(h->model, h->prec == CG_FP64 ? 0 : 1, h->tissue, h->variant,
+                                     h->d_states, h->P, h->d_gscale, a, s);
 }
 
 int batch_check(cg_ionic* const* hs, int nh, double dt_s)

@@ -78,8 +78,9 @@ struct ExplicitStep {
     double act_v = 0.0;
 };
 
-// Model kernels, one set per arithmetic type: _fp64 (IEEE double, model_fp64.hip) and
-// _fp32 (single precision with hardware reciprocal/exp2/log2, model_fp32.hip).
+// Model kernels, one set per arithmetic type: _fp64 (double, model_fp64.hip) and _fp32
+// (single precision with hardware reciprocal/exp2/log2, model_fp32.hip); the adaptive
+// solvers' kernels (_ode) in model_fp64_ode.hip and model_fp32_ode.hip.
 #define CG_DECLARE_MODEL_ENTRIES(SFX)                                                      \
     /* ionic step (tissue mode) on SoA states; Vm in V, Im in V/s */                       \
     hipError_t launch_ionic_tissue_##SFX(int model, int tissue, void* states, int64_t n,   \
@@ -109,6 +110,8 @@ struct ExplicitStep {
 
 CG_DECLARE_MODEL_ENTRIES(fp64)
 CG_DECLARE_MODEL_ENTRIES(fp32)
+CG_DECLARE_MODEL_ENTRIES(fp64_ode)
+CG_DECLARE_MODEL_ENTRIES(fp32_ode)
 
 // detector state, FP64 SoA [field][lane]
 enum {
@@ -161,12 +164,14 @@ struct BatchArgs {
 };
 
 // batched single-cell protocol launch (batch_kernels.hpp); variant = kernel shape
-hipError_t launch_cells_protocol_fp64(int model, int tissue, int variant, void* states,
-                                      const ModelParams& P, const void* gscale,
-                                      const BatchArgs& a, hipStream_t s);
-hipError_t launch_cells_protocol_fp32(int model, int tissue, int variant, void* states,
-                                      const ModelParams& P, const void* gscale,
-                                      const BatchArgs& a, hipStream_t s);
+#define CG_DECLARE_BATCH_ENTRY(SFX)                                                        \
+    hipError_t launch_cells_protocol_##SFX(int model, int tissue, int variant, void* states, \
+                                           const ModelParams& P, const void* gscale,       \
+                                           const BatchArgs& a, hipStream_t s);
+CG_DECLARE_BATCH_ENTRY(fp64)
+CG_DECLARE_BATCH_ENTRY(fp32)
+CG_DECLARE_BATCH_ENTRY(fp64_ode)
+CG_DECLARE_BATCH_ENTRY(fp32_ode)
 constexpr int BATCH_VARIANTS = 6;
 const char* batch_variant_name(int v);
 
@@ -177,7 +182,9 @@ inline hipError_t launch_ionic_tissue(int model, int prec, int tissue, void* sta
                                       const OdeArgs& ode, hipStream_t s)
 {
     if (n <= 0) return hipSuccess;
-    return (prec ? launch_ionic_tissue_fp32 : launch_ionic_tissue_fp64)(
+    const bool ad = ode.method != 0;
+    return (prec ? (ad ? launch_ionic_tissue_fp32_ode : launch_ionic_tissue_fp32)
+                 : (ad ? launch_ionic_tissue_fp64_ode : launch_ionic_tissue_fp64))(
         model, tissue, states, n, Vm, Im, dt_model, P, gscale, ode, s);
 }
 
@@ -188,7 +195,9 @@ inline hipError_t launch_ionic_cells(int model, int prec, int tissue, void* stat
                                      double* trace = nullptr, int64_t tcell = -1)
 {
     if (n <= 0 || n_steps <= 0) return hipSuccess;
-    return (prec ? launch_ionic_cells_fp32 : launch_ionic_cells_fp64)(
+    const bool ad = ode.method != 0;
+    return (prec ? (ad ? launch_ionic_cells_fp32_ode : launch_ionic_cells_fp32)
+                 : (ad ? launch_ionic_cells_fp64_ode : launch_ionic_cells_fp64))(
         model, tissue, states, n, t0_model, dt_model, n_steps, P, gscale, stim, ode, trace,
         tcell, s);
 }
@@ -199,7 +208,9 @@ inline hipError_t launch_explicit_hex(int model, int prec, int tissue, const Hex
                                       uint8_t* flag, double* tact, const ExplicitStep& st,
                                       const ModelParams& P, hipStream_t s)
 {
-    return (prec ? launch_explicit_hex_fp32 : launch_explicit_hex_fp64)(
+    const bool ad = st.ode.method != 0;
+    return (prec ? (ad ? launch_explicit_hex_fp32_ode : launch_explicit_hex_fp32)
+                 : (ad ? launch_explicit_hex_fp64_ode : launch_explicit_hex_fp64))(
         model, tissue, g, a, states, V, Vold, Vnew, Iion, flag, tact, st, P, s);
 }
 
@@ -208,8 +219,20 @@ inline hipError_t launch_ionic_rhs(int model, int prec, int tissue, const HexGeo
                                    double* x0, double* Iion, double* b,
                                    const ExplicitStep& st, const ModelParams& P, hipStream_t s)
 {
-    return (prec ? launch_ionic_rhs_fp32 : launch_ionic_rhs_fp64)(
+    const bool ad = st.ode.method != 0;
+    return (prec ? (ad ? launch_ionic_rhs_fp32_ode : launch_ionic_rhs_fp32)
+                 : (ad ? launch_ionic_rhs_fp64_ode : launch_ionic_rhs_fp64))(
         model, tissue, g, states, Vn, Vm1, x0, Iion, b, st, P, s);
+}
+
+inline hipError_t launch_cells_protocol(int model, int prec, int tissue, int variant,
+                                        void* states, const ModelParams& P,
+                                        const void* gscale, const BatchArgs& a, hipStream_t s)
+{
+    const bool ad = a.method != 0;
+    return (prec ? (ad ? launch_cells_protocol_fp32_ode : launch_cells_protocol_fp32)
+                 : (ad ? launch_cells_protocol_fp64_ode : launch_cells_protocol_fp64))(
+        model, tissue, variant, states, P, gscale, a, s);
 }
 
 } // namespace cg

@@ -6,10 +6,10 @@
 #include "model_kernels.hpp"
 
 namespace cg {
-CG_DEFINE_MODEL_ENTRIES(float, fp32)
+CG_DEFINE_MODEL_ENTRIES(float, false, fp32)
 } // namespace cg
 
 #include "batch_kernels.hpp"
 namespace cg {
-CG_DEFINE_BATCH_ENTRY(float, fp32)
+CG_DEFINE_BATCH_ENTRY(float, false, fp32)
 } // namespace cg

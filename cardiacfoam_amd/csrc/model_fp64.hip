@@ -3,12 +3,12 @@
 #include "model_kernels.hpp"
 
 namespace cg {
-CG_DEFINE_MODEL_ENTRIES(double, fp64)
+CG_DEFINE_MODEL_ENTRIES(double, false, fp64)
 } // namespace cg
 
 #include "batch_kernels.hpp"
 namespace cg {
-CG_DEFINE_BATCH_ENTRY(double, fp64)
+CG_DEFINE_BATCH_ENTRY(double, false, fp64)
 
 // Early-stroke classification and APD90/DI of each cell's beat records
 // (classify_early_strokes and compute_apd_di of postProcessing_restCurves.py:203-297):

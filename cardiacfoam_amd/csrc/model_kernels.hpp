@@ -423,13 +423,16 @@ __global__ __launch_bounds__(MBS) void k_ionic_eval(int tissue, int64_t n,
 }
 
 // ---------------------------------------------------------------- launchers
+// ADAPTIVE: the kernels of the adaptive solvers (ode.method 1 or 2), else Rush-Larsen.
+// Each set is instantiated in a translation unit of its own: the stage arrays of the
+// adaptive kernels take most of the compile time.
 inline unsigned grid_8(int64_t n, int bs)
 {
     int64_t nb = (n + bs - 1) / bs;
     return (unsigned)((nb + 7) / 8 * 8);  // multiple of 8 for the XCD remap
 }
 
-template <class T> struct ModelLaunch {
+template <class T, bool ADAPTIVE> struct ModelLaunch {
     template <class M>
     static hipError_t tissue(int tissue, void* states, int64_t n, const double* Vm, double* Im,
                              double dt_model, const ModelParams& P, const void* gscale,
@@ -439,9 +442,9 @@ template <class T> struct ModelLaunch {
 #define CG_IONIC_TISSUE(I)                                                                 \
     hipLaunchKernelGGL((k_ionic_tissue<M, T, I>), dim3(grid), dim3(MBS), 0, s, (T*)states, \
                        n, Vm, Im, T(dt_model), kparams<T>(P), (const T*)gscale, tissue, ode)
-        if (ode.method == 2) CG_IONIC_TISSUE(2);
-        else if (ode.method == 1) CG_IONIC_TISSUE(1);
-        else CG_IONIC_TISSUE(0);
+        if constexpr (!ADAPTIVE) CG_IONIC_TISSUE(0);
+        else if (ode.method == 2) CG_IONIC_TISSUE(2);
+        else CG_IONIC_TISSUE(1);
 #undef CG_IONIC_TISSUE
         return hipGetLastError();
     }
@@ -456,9 +459,9 @@ template <class T> struct ModelLaunch {
     hipLaunchKernelGGL((k_ionic_cells<M, T, I>), dim3(grid), dim3(MBS), 0, s, (T*)states,  \
                        n, t0, T(dt), n_steps, kparams<T>(P), (const T*)gscale, tissue, stim, \
                        ode, trace, tcell)
-        if (ode.method == 2) CG_IONIC_CELLS(2);
-        else if (ode.method == 1) CG_IONIC_CELLS(1);
-        else CG_IONIC_CELLS(0);
+        if constexpr (!ADAPTIVE) CG_IONIC_CELLS(0);
+        else if (ode.method == 2) CG_IONIC_CELLS(2);
+        else CG_IONIC_CELLS(1);
 #undef CG_IONIC_CELLS
         return hipGetLastError();
     }
@@ -473,15 +476,15 @@ template <class T> struct ModelLaunch {
 #define CG_EXPLICIT_HEX(U, I)                                                              \
     hipLaunchKernelGGL((k_explicit_hex<M, T, U, I>), dim3(grid), dim3(MBS), 0, s, g, a,    \
                        (T*)states, V, Vold, Vnew, Iion, flag, tact, st, kparams<T>(P), tissue)
-        if (st.ode.method == 2) {
-            if (a.fx) CG_EXPLICIT_HEX(false, 2);
-            else CG_EXPLICIT_HEX(true, 2);
-        } else if (st.ode.method == 1) {
-            if (a.fx) CG_EXPLICIT_HEX(false, 1);
-            else CG_EXPLICIT_HEX(true, 1);
-        } else {
+        if constexpr (!ADAPTIVE) {
             if (a.fx) CG_EXPLICIT_HEX(false, 0);
             else CG_EXPLICIT_HEX(true, 0);
+        } else if (st.ode.method == 2) {
+            if (a.fx) CG_EXPLICIT_HEX(false, 2);
+            else CG_EXPLICIT_HEX(true, 2);
+        } else {
+            if (a.fx) CG_EXPLICIT_HEX(false, 1);
+            else CG_EXPLICIT_HEX(true, 1);
         }
 #undef CG_EXPLICIT_HEX
         return hipGetLastError();
@@ -496,39 +499,39 @@ template <class T> struct ModelLaunch {
 #define CG_IONIC_RHS(I)                                                                    \
     hipLaunchKernelGGL((k_ionic_rhs<M, T, I>), dim3(grid_8(n, MBS)), dim3(MBS), 0, s, g,    \
                        (T*)states, Vn, Vm1, x0, Iion, b, st, kparams<T>(P), tissue)
-        if (st.ode.method == 2) CG_IONIC_RHS(2);
-        else if (st.ode.method == 1) CG_IONIC_RHS(1);
-        else CG_IONIC_RHS(0);
+        if constexpr (!ADAPTIVE) CG_IONIC_RHS(0);
+        else if (st.ode.method == 2) CG_IONIC_RHS(2);
+        else CG_IONIC_RHS(1);
 #undef CG_IONIC_RHS
         return hipGetLastError();
     }
 };
 
-// switch over the models for one arithmetic type
-#define CG_MODEL_SWITCH(T, FN, ...)                                                        \
+// switch over the models for one arithmetic type and solver family
+#define CG_MODEL_SWITCH(T, AD, FN, ...)                                                    \
     switch (model) {                                                                       \
-    case MODEL_BO: return ModelLaunch<T>::template FN<BuenoOrovio>(__VA_ARGS__);           \
-    case MODEL_TNNP: return ModelLaunch<T>::template FN<TNNP>(__VA_ARGS__);                \
-    case MODEL_ORD: return ModelLaunch<T>::template FN<ORd>(__VA_ARGS__);                  \
-    case MODEL_AP: return ModelLaunch<T>::template FN<AlievPanfilov>(__VA_ARGS__);         \
-    case MODEL_FDA: return ModelLaunch<T>::template FN<FdaManufactured>(__VA_ARGS__);      \
-    case MODEL_CRN: return ModelLaunch<T>::template FN<Courtemanche>(__VA_ARGS__);         \
-    case MODEL_PYS: return ModelLaunch<T>::template FN<PerisYague>(__VA_ARGS__);           \
-    case MODEL_STW: return ModelLaunch<T>::template FN<Stewart>(__VA_ARGS__);              \
-    case MODEL_GRD: return ModelLaunch<T>::template FN<Grandi>(__VA_ARGS__);               \
-    case MODEL_TOR: return ModelLaunch<T>::template FN<ToRORd>(__VA_ARGS__);               \
-    case MODEL_GAUR: return ModelLaunch<T>::template FN<Gaur>(__VA_ARGS__);                \
+    case MODEL_BO: return ModelLaunch<T, AD>::template FN<BuenoOrovio>(__VA_ARGS__);       \
+    case MODEL_TNNP: return ModelLaunch<T, AD>::template FN<TNNP>(__VA_ARGS__);            \
+    case MODEL_ORD: return ModelLaunch<T, AD>::template FN<ORd>(__VA_ARGS__);              \
+    case MODEL_AP: return ModelLaunch<T, AD>::template FN<AlievPanfilov>(__VA_ARGS__);     \
+    case MODEL_FDA: return ModelLaunch<T, AD>::template FN<FdaManufactured>(__VA_ARGS__);  \
+    case MODEL_CRN: return ModelLaunch<T, AD>::template FN<Courtemanche>(__VA_ARGS__);     \
+    case MODEL_PYS: return ModelLaunch<T, AD>::template FN<PerisYague>(__VA_ARGS__);       \
+    case MODEL_STW: return ModelLaunch<T, AD>::template FN<Stewart>(__VA_ARGS__);          \
+    case MODEL_GRD: return ModelLaunch<T, AD>::template FN<Grandi>(__VA_ARGS__);           \
+    case MODEL_TOR: return ModelLaunch<T, AD>::template FN<ToRORd>(__VA_ARGS__);           \
+    case MODEL_GAUR: return ModelLaunch<T, AD>::template FN<Gaur>(__VA_ARGS__);            \
     default: return hipErrorInvalidValue;                                                  \
     }
 
-// defines the four per-precision entry points of cg_internal.hpp for type T, suffix SFX
-#define CG_DEFINE_MODEL_ENTRIES(T, SFX)                                                    \
+// defines the four entry points of cg_internal.hpp for type T and solver family AD, suffix SFX
+#define CG_DEFINE_MODEL_ENTRIES(T, AD, SFX)                                                \
     hipError_t launch_ionic_tissue_##SFX(int model, int tissue, void* states, int64_t n,   \
                                          const double* Vm, double* Im, double dt_model,    \
                                          const ModelParams& P, const void* gscale,         \
                                          const OdeArgs& ode, hipStream_t s)                \
     {                                                                                      \
-        CG_MODEL_SWITCH(T, tissue, tissue, states, n, Vm, Im, dt_model, P, gscale, ode, s) \
+        CG_MODEL_SWITCH(T, AD, tissue, tissue, states, n, Vm, Im, dt_model, P, gscale, ode, s) \
     }                                                                                      \
     hipError_t launch_ionic_cells_##SFX(int model, int tissue, void* states, int64_t n,    \
                                         double t0, double dt, int n_steps,                 \
@@ -536,7 +539,7 @@ template <class T> struct ModelLaunch {
                                         const Stimulus& stim, const OdeArgs& ode,          \
                                         double* trace, int64_t tcell, hipStream_t s)       \
     {                                                                                      \
-        CG_MODEL_SWITCH(T, cells, tissue, states, n, t0, dt, n_steps, P, gscale, stim,     \
+        CG_MODEL_SWITCH(T, AD, cells, tissue, states, n, t0, dt, n_steps, P, gscale, stim, \
                         ode, trace, tcell, s)                                              \
     }                                                                                      \
     hipError_t launch_explicit_hex_##SFX(int model, int tissue, const HexGeom& g,          \
@@ -546,7 +549,7 @@ template <class T> struct ModelLaunch {
                                          const ExplicitStep& st, const ModelParams& P,     \
                                          hipStream_t s)                                    \
     {                                                                                      \
-        CG_MODEL_SWITCH(T, explicit_hex, tissue, g, a, states, V, Vold, Vnew, Iion, flag,  \
+        CG_MODEL_SWITCH(T, AD, explicit_hex, tissue, g, a, states, V, Vold, Vnew, Iion, flag, \
                         tact, st, P, s)                                                    \
     }                                                                                      \
     hipError_t launch_ionic_rhs_##SFX(int model, int tissue, const HexGeom& g,             \
@@ -555,7 +558,7 @@ template <class T> struct ModelLaunch {
                                       const ExplicitStep& st, const ModelParams& P,        \
                                       hipStream_t s)                                       \
     {                                                                                      \
-        CG_MODEL_SWITCH(T, ionic_rhs, tissue, g, states, Vn, Vm1, x0, Iion, b, st, P, s)   \
+        CG_MODEL_SWITCH(T, AD, ionic_rhs, tissue, g, states, Vn, Vm1, x0, Iion, b, st, P, s) \
     }
 
 } // namespace cg
