@@ -326,7 +326,7 @@ template <class T, bool ADAPTIVE> struct BatchLaunch {
                                            const BatchArgs& a, hipStream_t s)              \
     {                                                                                      \
         switch (model) {                                                                   \
-        case MODEL_BO: return BatchLaunch<T, AD>::variant<BuenoOrovio>(variant, tissue, states, P, gscale, a, s); \
+        case MODEL_BO: return BatchLaunch<arith_t<BuenoOrovio, T>, AD>::template variant<BuenoOrovio>(variant, tissue, states, P, gscale, a, s); \
         case MODEL_TNNP: return BatchLaunch<T, AD>::variant<TNNP>(variant, tissue, states, P, gscale, a, s); \
         case MODEL_ORD: return BatchLaunch<T, AD>::variant<ORd>(variant, tissue, states, P, gscale, a, s); \
         case MODEL_AP: return BatchLaunch<T, AD>::variant<AlievPanfilov>(variant, tissue, states, P, gscale, a, s); \
@@ -335,7 +335,7 @@ template <class T, bool ADAPTIVE> struct BatchLaunch {
         case MODEL_STW: return BatchLaunch<T, AD>::variant<Stewart>(variant, tissue, states, P, gscale, a, s); \
         case MODEL_GRD: return BatchLaunch<T, AD>::variant<Grandi>(variant, tissue, states, P, gscale, a, s); \
         case MODEL_TOR: return BatchLaunch<T, AD>::variant<ToRORd>(variant, tissue, states, P, gscale, a, s); \
-        case MODEL_GAUR: return BatchLaunch<T, AD>::variant<Gaur>(variant, tissue, states, P, gscale, a, s); \
+        case MODEL_GAUR: return BatchLaunch<arith_t<Gaur, T>, AD>::template variant<Gaur>(variant, tissue, states, P, gscale, a, s); \
         default: return hipErrorInvalidValue;                                              \
         }                                                                                  \
     }

@@ -41,7 +41,7 @@ struct BuenoOrovio {
     template <class T> CG_HD static T jion(T u, const T* y, const T* p)
     {
         const bool Hv = pos(u - p[thv]), Hw = pos(u - p[thw]), Ho = pos(u - p[tho]);
-        const T tso = p[tso1] + (p[tso2] - p[tso1]) * (T(1) + ctanh(p[kso] * (u - p[uso]))) / T(2);
+        const T tso = p[tso1] + (p[tso2] - p[tso1]) * half_1p_tanh(p[kso] * (u - p[uso]));
         const T to = Ho ? p[to2] : p[to1];
         const T jfi = Hv ? -y[1] * (u - p[thv]) * (p[uu] - u) / p[tfi] : T(0);
         const T jso = Hw ? T(1) / tso : (u - p[uo]) / to;
@@ -59,11 +59,11 @@ struct BuenoOrovio {
         const T vinf = Hv ? T(0) : (pos(p[thvm] - u) ? T(1) : T(0));
         const T tv = Hv ? p[tvp] : (Hvm ? p[tv2m] : p[tv1m]);
         // w: relaxes to 0 with tau_w+ above theta_w, else to w_inf with tau_w-
-        const T twm = p[tw1m] + (p[tw2m] - p[tw1m]) * (T(1) + ctanh(p[kwm] * (u - p[uwm]))) / T(2);
+        const T twm = p[tw1m] + (p[tw2m] - p[tw1m]) * half_1p_tanh(p[kwm] * (u - p[uwm]));
         const T winf = Hw ? T(0) : (Ho ? p[winfstar] : T(1) - u / p[twinf]);
         const T tw = Hw ? p[twp] : twm;
         // s
-        const T sinf = (T(1) + ctanh(p[ks] * (u - p[us]))) / T(2);
+        const T sinf = half_1p_tanh(p[ks] * (u - p[us]));
         const T ts = Hw ? p[ts2] : p[ts1];
         out.gate(1, vinf, tv);
         out.gate(2, winf, tw);

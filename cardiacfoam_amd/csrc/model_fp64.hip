@@ -1,14 +1,14 @@
-// FP64 instantiations of the model kernels (IEEE division, exp and log): the plain
+// FP64 instantiations of the model kernels (division as cg_f64.hpp): the plain
 // double-precision path of the tissue step and of the single-cell runs.
 #include "model_kernels.hpp"
 
 namespace cg {
-CG_DEFINE_MODEL_ENTRIES(double, false, fp64)
+CG_DEFINE_MODEL_ENTRIES(F64, false, fp64)
 } // namespace cg
 
 #include "batch_kernels.hpp"
 namespace cg {
-CG_DEFINE_BATCH_ENTRY(double, false, fp64)
+CG_DEFINE_BATCH_ENTRY(F64, false, fp64)
 
 // Early-stroke classification and APD90/DI of each cell's beat records
 // (classify_early_strokes and compute_apd_di of postProcessing_restCurves.py:203-297):
@@ -80,7 +80,7 @@ static hipError_t eval_of(int tissue, int64_t n, const double* st, const double*
                           const double* gsc, double* out, hipStream_t s)
 {
     hipLaunchKernelGGL(k_ionic_eval<M>, dim3((unsigned)((n + MBS - 1) / MBS)), dim3(MBS), 0, s,
-                       tissue, n, st, t, kind, solve_v, stim, kparams<double>(P), gsc, out);
+                       tissue, n, st, t, kind, solve_v, stim, kparams<arith_t<M, F64>>(P), gsc, out);
     return hipGetLastError();
 }
 

@@ -15,6 +15,22 @@ namespace cg {
 
 constexpr int MBS = 256;  // threads per block of the model kernels
 
+// Arithmetic type of model M where the kernels ask for T: F64 (cheap division) for the
+// FP64 Rush-Larsen kernels, except Gaur's, whose device code in it runs off the oracle
+// while the same source on the host agrees to 1e-9 (as its FP64 RKF45 kernel does, which
+// is refused); plain double for the adaptive solvers, whose stage arrays fill the registers
+// either way and compile three times longer in F64, except BuenoOrovio's.
+template <class M, class T> struct ArithOf {
+    using type = T;
+};
+template <> struct ArithOf<Gaur, F64> {
+    using type = double;
+};
+template <> struct ArithOf<BuenoOrovio, double> {
+    using type = F64;
+};
+template <class M, class T> using arith_t = typename ArithOf<M, T>::type;
+
 // model constants already in the kernel's arithmetic type (no per-lane conversions)
 template <class T> struct KParams {
     T p[MAX_PARAMS];
@@ -40,6 +56,12 @@ CG_DEV void store_states(const T (&y)[NS], T* __restrict__ st, int64_t n, int64_
     T* sp = st + c + first * n;
 #pragma unroll
     for (int q = first; q < NS; ++q, sp += n) *sp = y[q];
+}
+
+// the model's V variable from Vm (V)
+template <class M, class T> CG_DEV T model_v(double vm)
+{
+    return T(double(F64(vm * M::VMUL + M::VOFF) / F64(M::VSCALE)));
 }
 
 // States of model M in the handle's storage (offsets from StateRef on FP32 handles):
@@ -169,7 +191,7 @@ __global__ __launch_bounds__(MBS) void k_ionic_tissue(T* __restrict__ st, int64_
     }
     T y[M::NS], sw[M::NS];
     load_model_states<M>(y, sw, st, n, i, 1);
-    const T v = T((Vm[i] * M::VMUL + M::VOFF) / M::VSCALE);
+    const T v = model_v<M, T>(Vm[i]);
     const T I = tissue_advance<M, T, INTEG>(v, y, sw, dt, p, tissue, gs, ode, i);
     store_states(sw, st, n, i, 1);
     Im[i] = double(I) * M::ISCALE;
@@ -315,7 +337,7 @@ __global__ __launch_bounds__(MBS) void k_explicit_hex(
     T y[M::NS], sw[M::NS];
     load_model_states<M>(y, sw, st, n, c, 1);
     const double vn = V[c];
-    const T v = T((vn * M::VMUL + M::VOFF) / M::VSCALE);
+    const T v = model_v<M, T>(vn);
     const T I = tissue_advance<M, T, INTEG>(v, y, sw, T(s.dt_model), p, tissue, one, s.ode, c);
     store_states(sw, st, n, c, 1);
     const double iion = double(I) * M::ISCALE;
@@ -342,11 +364,12 @@ __global__ __launch_bounds__(MBS) void k_explicit_hex(
 // gate (s.gate) the launch may be queued before the previous step's solve is known to have
 // converged: it then does nothing unless the solver recorded the expected generation.
 // waves per SIMD the register allocation of k_ionic_rhs aims at (1: the compiler's
-// choice).  FP64 ORd: 2, at 256 VGPRs with 296 B/lane of spills instead of 256 + 84 AGPRs
-// at one wave; measured 4.6 % faster per implicit 2.1M-cell FP64 step (0.938 vs 0.983 ms).
+// choice).  FP64 ORd: 2, at 256 VGPRs with 152 B/lane of spills where one wave takes 256 +
+// 62 AGPRs; with the spills of an earlier build (296 B) it was 4.6 % faster per implicit
+// 2.1M-cell FP64 step.  Grandi (256 + 4 AGPRs at one wave) likewise.
 template <class M, class T> constexpr int rhs_waves()
 {
-    if constexpr (std::is_same_v<M, ORd> && sizeof(T) == 8) return 2;
+    if constexpr ((std::is_same_v<M, ORd> || std::is_same_v<M, Grandi>) && sizeof(T) == 8) return 2;
     return 1;
 }
 
@@ -374,7 +397,7 @@ void k_ionic_rhs(HexGeom g, T* __restrict__ st,
     // behind it
     const double vo = (x0 || s.c00 != 0.0 || s.act_flag) ? Vm1[c] : 0.0;
     const uint8_t fl = s.act_flag ? s.act_flag[c] : 0;
-    const T v = T((vn * M::VMUL + M::VOFF) / M::VSCALE);
+    const T v = model_v<M, T>(vn);
     const T I = tissue_advance<M, T, INTEG>(v, y, sw, T(s.dt_model), p, tissue, one, s.ode, c);
     store_states(sw, st, n, c, 1);
     const double iion = double(I) * M::ISCALE;
@@ -398,27 +421,28 @@ __global__ __launch_bounds__(MBS) void k_ionic_eval(int tissue, int64_t n,
                                                     const double* __restrict__ st,
                                                     const double* __restrict__ t, int kind,
                                                     int solve_v, Stimulus stim,
-                                                    KParams<double> P,
+                                                    KParams<arith_t<M, F64>> P,
                                                     const double* __restrict__ gsc,
                                                     double* __restrict__ out)
 {
+    using T = arith_t<M, F64>;
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    const double* p = P.p;
-    double gs[4] = {1.0, 1.0, 1.0, 1.0};
+    const T* p = P.p;
+    T gs[4] = {1.0, 1.0, 1.0, 1.0};
     if (gsc)
         for (int k = 0; k < 4; ++k) gs[k] = gsc[k * n + i];
-    double y[M::NS];
+    T y[M::NS];
     for (int q = 0; q < M::NS; ++q) y[q] = st[q * n + i];
-    const double istim = solve_v ? stimulus_current(t[i], stim) : 0.0;
+    const T istim = solve_v ? stimulus_current(t[i], stim) : 0.0;
     if (kind == 0) {
-        double d[M::NS];
+        T d[M::NS];
         Ops<M>::deriv(y, d, p, tissue, gs, solve_v != 0, istim, Ops<M>::vt(y[0], p));
-        for (int q = 0; q < M::NS; ++q) out[q * n + i] = d[q];
+        for (int q = 0; q < M::NS; ++q) out[q * n + i] = double(d[q]);
     } else if constexpr (Algebraic<M>::NA > 0) {
-        double a[Algebraic<M>::NA];
+        T a[Algebraic<M>::NA];
         Algebraic<M>::eval(y, p, istim, a);
-        for (int q = 0; q < Algebraic<M>::NA; ++q) out[q * n + i] = a[q];
+        for (int q = 0; q < Algebraic<M>::NA; ++q) out[q * n + i] = double(a[q]);
     }
 }
 
@@ -510,7 +534,8 @@ template <class T, bool ADAPTIVE> struct ModelLaunch {
 // switch over the models for one arithmetic type and solver family
 #define CG_MODEL_SWITCH(T, AD, FN, ...)                                                    \
     switch (model) {                                                                       \
-    case MODEL_BO: return ModelLaunch<T, AD>::template FN<BuenoOrovio>(__VA_ARGS__);       \
+    case MODEL_BO:                                                                         \
+        return ModelLaunch<arith_t<BuenoOrovio, T>, AD>::template FN<BuenoOrovio>(__VA_ARGS__); \
     case MODEL_TNNP: return ModelLaunch<T, AD>::template FN<TNNP>(__VA_ARGS__);            \
     case MODEL_ORD: return ModelLaunch<T, AD>::template FN<ORd>(__VA_ARGS__);              \
     case MODEL_AP: return ModelLaunch<T, AD>::template FN<AlievPanfilov>(__VA_ARGS__);     \
@@ -520,7 +545,8 @@ template <class T, bool ADAPTIVE> struct ModelLaunch {
     case MODEL_STW: return ModelLaunch<T, AD>::template FN<Stewart>(__VA_ARGS__);          \
     case MODEL_GRD: return ModelLaunch<T, AD>::template FN<Grandi>(__VA_ARGS__);           \
     case MODEL_TOR: return ModelLaunch<T, AD>::template FN<ToRORd>(__VA_ARGS__);           \
-    case MODEL_GAUR: return ModelLaunch<T, AD>::template FN<Gaur>(__VA_ARGS__);            \
+    case MODEL_GAUR:                                                                       \
+        return ModelLaunch<arith_t<Gaur, T>, AD>::template FN<Gaur>(__VA_ARGS__);          \
     default: return hipErrorInvalidValue;                                                  \
     }
 

@@ -220,3 +220,30 @@ def test_coupling_signals_and_io_states(gpu, orc):
     v = tn.stateVariableValues(7)
     assert v.shape == (len(names),) and v[0] == pytest.approx(Vm_next[7] * 1000.0, rel=1e-15)
     np.testing.assert_array_equal(v[1:], S[1:, 7])
+
+
+@pytest.mark.parametrize("name", ["BO_epi", "AP", "TNNP_M", "ORd", "CRN", "PYS", "STW", "GRD",
+                                  "TOR_M", "GAUR"])
+def test_rates_far_outside_the_physiological_range(gpu, orc, name):
+    """Rates at potentials whose exponentials overflow, vanish or are undefined: infinities
+    and NaN where the oracle's IEEE division has them, 1e-10 relative elsewhere (an
+    exponential of 1000 mV / 0.2 mV carries the rounding of its argument, 5000 * 1.1e-16,
+    and a rate sums a few dozen such terms)."""
+    _say("eval far from rest", name)
+    m, tis, key, word, _ = MODELS[name]
+    V = np.array([-1000.0, -300.0, -150.0, -0.0, 0.25, 150.0, 300.0, 1000.0, np.inf, -np.inf,
+                  np.nan])
+    if name.startswith("BO"):        # the oracle multiplies by its Heavisides: 0 * inf there
+        V = V[~np.isinf(V)]
+    n = V.size
+    c, S, _ = physiological_states(orc, name, n, seed=5)
+    S[0] = V / (85.7 if name.startswith("BO") else 100.0 if name == "AP" else 1.0)
+    R, _ = _oracle_rows(orc, m, tis, c, S, np.zeros(n), False, None)
+    got = gpu.IonicModel(key, word, n).eval("rates", S)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(R))
+    np.testing.assert_array_equal(np.isinf(got), np.isinf(R))
+    fin = np.isfinite(R)
+    scale = np.maximum(np.abs(R), np.max(np.abs(np.where(fin, R, 0.0)), axis=1, keepdims=True)
+                       * 1e-6)
+    _say("  max relative error %.3e" % np.max(np.abs(got[fin] - R[fin]) / (scale[fin] + 1e-300)))
+    assert np.all(np.abs(got[fin] - R[fin]) <= 1e-10 * scale[fin] + 1e-300)
