@@ -1,14 +1,24 @@
 // Deterministic grid reductions without atomics or device-scope fences: every reducing
-// kernel runs RG blocks of RBS threads over contiguous chunks and writes one partial per
-// block; the consumer kernel sums the RG partials in a fixed order in every block, so all
-// blocks see bit-identical scalars and take identical decisions.
+// kernel runs up to RG blocks of RBS threads over contiguous chunks and writes one partial
+// per block; the consumer kernel (launched on as many blocks) sums the partials in a fixed
+// order in every block, so all blocks see bit-identical scalars and take identical
+// decisions.
 #pragma once
 #include "cg_common.hpp"
 
 namespace cg {
 
 constexpr int RBS = 256;   // reducing kernels (measured best with RG = 1024 on 2.1 M cells)
-constexpr int RG = 1024;   // blocks of every reducing kernel
+constexpr int RG = 1024;   // most blocks of a reducing kernel (stride of the partials' slots)
+
+// blocks of the reducing kernels over `items` (cells, or quads of cells): one item per lane
+// until RG blocks, so a small mesh launches and sums no idle blocks; a multiple of 8 for
+// the XCD remap.
+inline unsigned reduce_grid(int64_t items)
+{
+    const int64_t nb = ((items + RBS - 1) / RBS + 7) / 8 * 8;
+    return (unsigned)(nb < RG ? nb : RG);
+}
 
 template <int NT, int NV> CG_DEV void block_sum(double (&v)[NV])
 {
@@ -31,16 +41,20 @@ template <int NT, int NV> CG_DEV void block_sum(double (&v)[NV])
     __syncthreads();
 }
 
-// fixed-order sums of the RG partials of NV slots: the same values in every block
+// fixed-order sums of the nb partials of NV slots: the same values in every block
 template <int NV>
-CG_DEV void sum_slots(const double* __restrict__ part, const int (&slot)[NV], double (&v)[NV])
+CG_DEV void sum_slots(const double* __restrict__ part, const int (&slot)[NV], double (&v)[NV],
+                      int nb)
 {
     static_assert(RG % RBS == 0, "partials must split evenly over the block");
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
         v[k] = 0.0;
 #pragma unroll
-        for (int q = 0; q < RG / RBS; ++q) v[k] += part[slot[k] * RG + q * RBS + threadIdx.x];
+        for (int q = 0; q < RG / RBS; ++q) {
+            const int i = q * RBS + (int)threadIdx.x;
+            if (i < nb) v[k] += part[slot[k] * RG + i];
+        }
     }
     block_sum<RBS, NV>(v);
 }

@@ -70,9 +70,9 @@ CG_DEV double ell_rowsum(const EllView& E, int64_t i)
     return a;
 }
 
-// contiguous chunk of rows per block for the reducing kernels (RG blocks of RBS)
+// contiguous chunk of rows per block for the reducing kernels
 #define ROW_LOOP(N)                                                                        \
-    const int64_t chunk_ = (((N) + RG - 1) / RG + RBS - 1) / RBS * RBS;                    \
+    const int64_t chunk_ = (((N) + gridDim.x - 1) / gridDim.x + RBS - 1) / RBS * RBS;      \
     const int64_t lo_ = (int64_t)blockIdx.x * chunk_;                                      \
     const int64_t hi_ = lo_ + chunk_ < (N) ? lo_ + chunk_ : (N);                           \
     for (int64_t i = lo_ + threadIdx.x; i < hi_; i += RBS)
@@ -111,7 +111,7 @@ __global__ __launch_bounds__(RBS) void k_r0(EllView E, const double* __restrict_
                                             double* __restrict__ part)
 {
     double xs[1];
-    sum_slots<1>(part, {L_XS}, xs);
+    sum_slots<1>(part, {L_XS}, xs, gridDim.x);
     const double xref = xs[0] / double(E.n);
     double v[3] = {0.0, 0.0, 0.0};
     ROW_LOOP(E.n)
@@ -143,7 +143,7 @@ __global__ __launch_bounds__(RBS) void k_s(EllView E, const double* __restrict__
 {
     if (S->done_gen == gen) return;
     double v3[3];
-    sum_slots<3>(part, {L_G + (k & 1), L_L1 + (k & 1), L_NF}, v3);
+    sum_slots<3>(part, {L_G + (k & 1), L_L1 + (k & 1), L_NF}, v3, gridDim.x);
     const double l1 = v3[1], nf = v3[2] + 1e-20;
     const double l10 = k == 0 ? l1 : S->l1_0;
     const bool conv = l1 < tol * nf || (rel > 1e-20 && l1 < rel * l10);
@@ -182,7 +182,7 @@ __global__ __launch_bounds__(RBS) void k_u(EllView E, double* __restrict__ psi,
 {
     if (S->done_gen == gen) return;
     double v2[2];
-    sum_slots<2>(part, {L_G + (k & 1), L_D}, v2);
+    sum_slots<2>(part, {L_G + (k & 1), L_D}, v2, gridDim.x);
     const double gam = v2[0], del = v2[1];
     double alpha, beta = 0.0;
     if (k == 0) {
@@ -225,6 +225,7 @@ unsigned blocks_of(int64_t n) { return (unsigned)((n + EBS - 1) / EBS); }
 
 struct LduSolver {
     int64_t n = 0, nf = 0;
+    unsigned rgrid = RG;      // blocks of the reducing kernels
     int K = 0;
     int32_t* col = nullptr;
     int32_t* fidx = nullptr;
@@ -277,6 +278,7 @@ int ldu_create(LduSolver** out, int64_t n, int64_t nf, const int32_t* lower,
     }
     LduSolver* L = new LduSolver();
     L->n = n; L->nf = nf; L->K = K;
+    L->rgrid = reduce_grid(n);
     bool ok = true;
     auto A = [&](void** ptr, size_t bytes) { ok &= hipMalloc(ptr, bytes) == hipSuccess; };
     A((void**)&L->col, 4 * (size_t)K * n);
@@ -371,19 +373,19 @@ int ldu_solve(LduSolver* L, double* psi, const double* b, bool device, double to
     }
     const EllView E = L->view();
     const long long gen = ++L->gen;
-    hipLaunchKernelGGL(k_mean, dim3(RG), dim3(RBS), 0, L->stream, L->n, (const double*)dpsi, L->part);
-    hipLaunchKernelGGL(k_r0, dim3(RG), dim3(RBS), 0, L->stream, E, (const double*)dpsi, db,
+    hipLaunchKernelGGL(k_mean, dim3(L->rgrid), dim3(RBS), 0, L->stream, L->n, (const double*)dpsi, L->part);
+    hipLaunchKernelGGL(k_r0, dim3(L->rgrid), dim3(RBS), 0, L->stream, E, (const double*)dpsi, db,
                        L->r, L->u, L->part);
-    hipLaunchKernelGGL(k_s, dim3(RG), dim3(RBS), 0, L->stream, E, (const double*)L->u, L->z,
+    hipLaunchKernelGGL(k_s, dim3(L->rgrid), dim3(RBS), 0, L->stream, E, (const double*)L->u, L->z,
                        L->part, L->S, gen, 0, tol, rel, max_iter);
     int k = 0;
     for (;;) {
         // a chunk of iterations, then the 64-byte state; iterations after convergence
         // return at once
         for (int q = 0; q < 8; ++q, ++k) {
-            hipLaunchKernelGGL(k_u, dim3(RG), dim3(RBS), 0, L->stream, E, dpsi, L->r, L->u,
+            hipLaunchKernelGGL(k_u, dim3(L->rgrid), dim3(RBS), 0, L->stream, E, dpsi, L->r, L->u,
                                L->p, L->s, (const double*)L->z, L->part, L->S, gen, k);
-            hipLaunchKernelGGL(k_s, dim3(RG), dim3(RBS), 0, L->stream, E, (const double*)L->u,
+            hipLaunchKernelGGL(k_s, dim3(L->rgrid), dim3(RBS), 0, L->stream, E, (const double*)L->u,
                                L->z, L->part, L->S, gen, k + 1, tol, rel, max_iter);
         }
         if (hipMemcpyAsync(L->hS, L->S, sizeof(LduState), hipMemcpyDeviceToHost, L->stream) !=

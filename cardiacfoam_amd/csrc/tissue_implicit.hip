@@ -16,7 +16,9 @@
 //   fp64 path : CG in fp64 to ||b - A x||_2 <= tol ||b||_2.
 //   mixed path: iterative refinement; residual and solution in fp64, each correction from
 //               an fp32 CG (fp32 operator and vectors, fp64 dot products) to 1e-4 relative.
-// Kernels of one step:
+// Where the matrix is diagonally dominant enough (below) both paths take Chebyshev's
+// iteration in place of the conjugate gradients; see k_cheb.
+// Kernels of one CG step:
 //   residual (first)  x0 = V^n, b += tensor correction, r = b - A x0, u = M^-1 r
 //   per iteration k   S: convergence test on r_k; w = A u, partial (w,u)
 //                     U: alpha, beta; p = u + beta p, s = w + beta s, x += alpha p,
@@ -38,6 +40,7 @@
 namespace cg {
 
 constexpr int BS = 256;    // elementwise kernels
+constexpr int SMALL_N = 8192;  // most cells of an FP64 solve that stays with the CG
 
 // partial-sum slots (RG doubles each)
 enum { P_G = 0,      // (r,u), parity sets 0 and 1
@@ -48,7 +51,8 @@ enum { P_G = 0,      // (r,u), parity sets 0 and 1
        P_L1 = 7,     // sum |r| (OpenFOAM norm), parity sets 7 and 8
        P_NF = 9,     // normalisation factor terms of the solve's first residual
        P_XS = 10,    // sum of the initial guess (its mean is OpenFOAM's xRef)
-       P_NSLOT = 11 };
+       P_RRI = 11,   // (r,r) of a Chebyshev solve's first residual (FP64 path)
+       P_NSLOT = 12 };
 
 enum { S_RR, S_BB, S_R0, S_NSCAL };
 struct DevState {
@@ -150,6 +154,8 @@ CG_DEV V4<T> apply_quad(const HexOp<T>& A, const T* __restrict__ x, int64_t c0, 
 // and of sigma_xy as 32-byte loads plus their end values, the y-gradients of the cells and
 // their x-neighbours and the x-gradients of the cells and their y-neighbours taken from
 // those rows.  Same walls (clamped neighbours) and the same expression order per cell.
+// LAY: sigma_xy is constant in the plane, oxy its nz values.
+template <bool LAY>
 CG_DEV V4<double> quad_correction_xy(const double* __restrict__ V,
                                      const double* __restrict__ oxy, int64_t c0, const IJK& q,
                                      const HexGeom& g)
@@ -160,8 +166,14 @@ CG_DEV V4<double> quad_correction_xy(const double* __restrict__ V,
     const V4<double> v0 = ld4(V + c0), vm = ld4(V + rm), vp = ld4(V + rp);
     const double v0l = V[c0 + xl], v0r = V[c0 + xr], vml = V[rm + xl], vmr = V[rm + xr];
     const double vpl = V[rp + xl], vpr = V[rp + xr];
-    const V4<double> o0 = ld4(oxy + c0), om = ld4(oxy + rm), op = ld4(oxy + rp);
-    const double o0l = oxy[c0 + xl], o0r = oxy[c0 + xr];
+    V4<double> o0, om, op;
+    double o0l, o0r;
+    if constexpr (LAY) {
+        o0 = om = op = o0l = o0r = oxy[q.k];
+    } else {
+        o0 = ld4(oxy + c0); om = ld4(oxy + rm); op = ld4(oxy + rp);
+        o0l = oxy[c0 + xl]; o0r = oxy[c0 + xr];
+    }
     const double rhx = 0.5 / g.hx, rhy = 0.5 / g.hy;
     // faces -x/+x (d = x, e = y): y-gradients at the cells and their x-neighbours
     const V4<double> gy = (vp - vm) * rhy;
@@ -179,6 +191,88 @@ CG_DEV V4<double> quad_correction_xy(const double* __restrict__ V,
     return 0.25 * qx * (2.0 * rhx) + 0.25 * qy * (2.0 * rhy);
 }
 
+// Layered coefficients: with a conductivity that is constant in each z-plane (uniform, or
+// fibres that rotate through the wall of a block) a_f comes from three numbers per plane
+// (lay [nz][3]) instead of three planes of n, the same numbers.
+template <class T> struct Layers {
+    const T* k3;   // fx, fy, fz of plane k; fz of the last plane 0
+    const T* od;   // sigma_xy of plane k (FP64), or null
+};
+
+// A x of four rows and their diagonal
+template <class T, bool LAY, class LD>
+CG_DEV V4<T> apply_quad_diag(const HexOp<T>& A, const Layers<T>& L, const LD& x, int64_t c0,
+                             const IJK& q, const HexGeom& g, V4<T>& xc, V4<T>& diag)
+{
+    const int64_t sy = g.nx, sz = (int64_t)g.nx * g.ny;
+    const int64_t ym = q.j > 0 ? c0 - sy : c0, yp = q.j < g.ny - 1 ? c0 + sy : c0;
+    const int64_t zm = q.k > 0 ? c0 - sz : c0, zp = q.k < g.nz - 1 ? c0 + sz : c0;
+    const int64_t xl = q.i > 0 ? c0 - 1 : c0, xr = q.i + 4 < g.nx ? c0 + 4 : c0 + 3;
+    xc = x.q4(c0);
+    const V4<T> xym = x.q4(ym), xyp = x.q4(yp), xzm = x.q4(zm), xzp = x.q4(zp);
+    const T x_l = x(xl), x_r = x(xr);
+    const V4<T> xxm = {x_l, xc.x, xc.y, xc.z};
+    const V4<T> xxp = {xc.y, xc.z, xc.w, x_r};
+    V4<T> fxp, fxm, fyp, fym, fzp, fzm;   // 0 on walls
+    if constexpr (LAY) {
+        const T fx = L.k3[3 * q.k], fy = L.k3[3 * q.k + 1];
+        const T l = q.i > 0 ? fx : T(0), r = q.i + 4 < g.nx ? fx : T(0);
+        const T ylo = q.j > 0 ? fy : T(0), yhi = q.j < g.ny - 1 ? fy : T(0);
+        const T zlo = q.k > 0 ? L.k3[3 * q.k - 1] : T(0), zhi = L.k3[3 * q.k + 2];
+        fxm = {l, fx, fx, fx};
+        fxp = {fx, fx, fx, r};
+        fym = ylo; fyp = yhi; fzm = zlo; fzp = zhi;
+    } else {
+        const V4<T> fx = ld4(A.fx + c0);
+        const T fl = A.fx[xl];
+        fxp = fx;
+        fxm = {q.i > 0 ? fl : T(0), fx.x, fx.y, fx.z};
+        fyp = ld4(A.fy + c0);
+        fzp = ld4(A.fz + c0);
+        fym = ld4(A.fy + ym);
+        fzm = ld4(A.fz + zm);
+        if (q.j == 0) fym = T(0);
+        if (q.k == 0) fzm = T(0);
+    }
+    diag = A.mass + ((fxp + fxm) + (fyp + fym) + (fzp + fzm));
+    return A.mass * xc + (fxp * (xc - xxp) + fxm * (xc - xxm)) +
+           (fyp * (xc - xyp) + fym * (xc - xym)) + (fzp * (xc - xzp) + fzm * (xc - xzm));
+}
+// the same for one row
+template <class T, bool LAY, class LD>
+CG_DEV T apply_row_diag(const HexOp<T>& A, const Layers<T>& L, const LD& x, int64_t c,
+                        const IJK& q, const HexGeom& g, T& xc, T& diag)
+{
+    const Nbr b = nbr_of(c, q, g);
+    xc = T(x(c));
+    T fxp, fxm, fyp, fym, fzp, fzm;
+    if constexpr (LAY) {
+        const T fx = L.k3[3 * q.k], fy = L.k3[3 * q.k + 1];
+        fxm = q.i > 0 ? fx : T(0);
+        fxp = q.i < g.nx - 1 ? fx : T(0);
+        fym = q.j > 0 ? fy : T(0);
+        fyp = q.j < g.ny - 1 ? fy : T(0);
+        fzm = q.k > 0 ? L.k3[3 * q.k - 1] : T(0);
+        fzp = L.k3[3 * q.k + 2];
+    } else {
+        fxp = A.fx[c]; fyp = A.fy[c]; fzp = A.fz[c];
+        fxm = q.i > 0 ? A.fx[b.xm] : T(0);
+        fym = q.j > 0 ? A.fy[b.ym] : T(0);
+        fzm = q.k > 0 ? A.fz[b.zm] : T(0);
+    }
+    diag = A.mass + ((fxp + fxm) + (fyp + fym) + (fzp + fzm));
+    return A.mass * xc + (fxp * (xc - T(x(b.xp))) + fxm * (xc - T(x(b.xm)))) +
+           (fyp * (xc - T(x(b.yp))) + fym * (xc - T(x(b.ym)))) +
+           (fzp * (xc - T(x(b.zp))) + fzm * (xc - T(x(b.zm))));
+}
+// r / d with the reciprocal's own accuracy (a preconditioner)
+CG_DEV float jacobi(float r, float d) { return r * __builtin_amdgcn_rcpf(d); }
+CG_DEV double jacobi(double r, double d) { return div_f64(r, d); }
+template <class T> CG_DEV V4<T> jacobi4(const V4<T>& r, const V4<T>& d)
+{
+    return V4<T>{jacobi(r.x, d.x), jacobi(r.y, d.y), jacobi(r.z, d.z), jacobi(r.w, d.w)};
+}
+
 // one cell per lane (elementwise kernels)
 #define CELL_INDEX                                                                         \
     const uint32_t bid = xcd_block(blockIdx.x, gridDim.x);                                 \
@@ -187,11 +281,19 @@ CG_DEV V4<double> quad_correction_xy(const double* __restrict__ V,
     if (c >= n) return;                                                                    \
     const IJK cc = ijk_of((uint32_t)c, g);
 
-// contiguous chunk of cells per block (reducing kernels on RG blocks of RBS threads)
+// contiguous chunk of cells per block (reducing kernels, blocks of RBS threads)
 #define RANGE_LOOP(g)                                                                      \
     const int64_t n = (int64_t)(g).nx * (g).ny * (g).nz;                                   \
     const uint32_t bid = xcd_block(blockIdx.x, gridDim.x);                                 \
-    const int64_t chunk_ = ((n + RG - 1) / RG + RBS - 1) / RBS * RBS;                      \
+    const int64_t chunk_ = ((n + gridDim.x - 1) / gridDim.x + RBS - 1) / RBS * RBS;                      \
+    const int64_t lo_ = (int64_t)bid * chunk_;                                             \
+    const int64_t hi_ = lo_ + chunk_ < n ? lo_ + chunk_ : n;                               \
+    for (int64_t c = lo_ + threadIdx.x; c < hi_; c += RBS)
+
+// the same with the block index already remapped (bid in scope)
+#define RANGE_LOOP_B(g)                                                                    \
+    const int64_t n = (int64_t)(g).nx * (g).ny * (g).nz;                                   \
+    const int64_t chunk_ = ((n + gridDim.x - 1) / gridDim.x + RBS - 1) / RBS * RBS;        \
     const int64_t lo_ = (int64_t)bid * chunk_;                                             \
     const int64_t hi_ = lo_ + chunk_ < n ? lo_ + chunk_ : n;                               \
     for (int64_t c = lo_ + threadIdx.x; c < hi_; c += RBS)
@@ -199,7 +301,7 @@ CG_DEV V4<double> quad_correction_xy(const double* __restrict__ V,
 // the same chunks in quads of 4 consecutive cells (c0 = 4 qi), for nx % 4 == 0
 #define RANGE_LOOP_Q(g)                                                                    \
     const int64_t nq_ = (int64_t)(g).nx * (g).ny * (g).nz / 4;                             \
-    const int64_t qchunk_ = ((nq_ + RG - 1) / RG + RBS - 1) / RBS * RBS;                   \
+    const int64_t qchunk_ = ((nq_ + gridDim.x - 1) / gridDim.x + RBS - 1) / RBS * RBS;                   \
     const int64_t qlo_ = (int64_t)bid * qchunk_;                                           \
     const int64_t qhi_ = qlo_ + qchunk_ < nq_ ? qlo_ + qchunk_ : nq_;                      \
     for (int64_t qi = qlo_ + threadIdx.x; qi < qhi_; qi += RBS)
@@ -234,8 +336,9 @@ __global__ __launch_bounds__(BS) void k_invdiag(HexGeom g, HexOp<T> A, T* __rest
 //   Block 0 adds the iterations of the previous solve to the running sum.
 //   OF: also sum |r| and the normalisation terms |A x - mass xref| + |b - mass xref|
 //   (lduMatrix::solver::normFactor; the row sums of A are the mass coefficient).
-template <class TP, class LD, bool CORR, bool OF>
-CG_DEV void residual_range(const HexGeom& g, const HexOp<double>& A, const TP* __restrict__ invd_t,
+template <class TP, class LD, bool CORR, bool OF, bool LAY>
+CG_DEV void residual_range(const HexGeom& g, const HexOp<double>& A, const Layers<double>& L,
+                           const TP* __restrict__ invd_t,
                            const LD& X, const double* __restrict__ xin, double* __restrict__ xout,
                            const double* bsrc, double* bout, const double* __restrict__ od,
                            unsigned od_mask, TP* __restrict__ rt, TP* __restrict__ ut,
@@ -249,10 +352,12 @@ CG_DEV void residual_range(const HexGeom& g, const HexOp<double>& A, const TP* _
         if (CORR) bc += hex_tensor_correction(xin, od, n, c, q.i, q.j, q.k, g, od_mask);
         if (bout) bout[c] = bc;
         if (xout) xout[c] = X(c);
-        const double ax = apply_row(A, X, c, q, g);
+        double xc, d;
+        const double ax = LAY ? apply_row_diag<double, true>(A, L, X, c, q, g, xc, d)
+                              : apply_row(A, X, c, q, g);
         const double r = bc - ax;
         const TP rr = TP(r);
-        const TP u = invd_t[c] * rr;
+        const TP u = LAY ? jacobi(rr, TP(d)) : invd_t[c] * rr;
         rt[c] = rr;
         ut[c] = u;
         v[0] += double(rr) * double(u);
@@ -267,8 +372,8 @@ CG_DEV void residual_range(const HexGeom& g, const HexOp<double>& A, const TP* _
 }
 
 // the same on quads of cells (nx % 4 == 0), the correction limited to sigma_xy (CORRXY)
-template <class TP, class LD, bool CORRXY, bool OF>
-CG_DEV void residual_range_q(const HexGeom& g, const HexOp<double>& A,
+template <class TP, class LD, bool CORRXY, bool OF, bool LAY>
+CG_DEV void residual_range_q(const HexGeom& g, const HexOp<double>& A, const Layers<double>& L,
                              const TP* __restrict__ invd_t, const LD& X,
                              const double* __restrict__ xin, double* __restrict__ xout,
                              const double* bsrc, double* bout, const double* __restrict__ oxy,
@@ -281,13 +386,17 @@ CG_DEV void residual_range_q(const HexGeom& g, const HexOp<double>& A,
         const int64_t c0 = qi * 4;
         const IJK q = ijk_of((uint32_t)c0, g);
         V4<double> bc = ld4(bsrc + c0);
-        if (CORRXY) bc += quad_correction_xy(xin, oxy, c0, q, g);
+        if (CORRXY) bc += quad_correction_xy<LAY>(xin, oxy, c0, q, g);
         if (bout) st4(bout + c0, bc);
         if (xout) st4(xout + c0, X.q4(c0));
-        const V4<double> ax = apply_quad_ld(A, X, c0, q, g);
+        V4<double> xc, d, ax;
+        if constexpr (LAY) ax = apply_quad_diag<double, true>(A, L, X, c0, q, g, xc, d);
+        else ax = apply_quad_ld(A, X, c0, q, g);
         const V4<double> r = bc - ax;
         const V4<TP> rr = __builtin_convertvector(r, V4<TP>);
-        const V4<TP> u = ld4(invd_t + c0) * rr;
+        V4<TP> u;
+        if constexpr (LAY) u = jacobi4<TP>(rr, __builtin_convertvector(d, V4<TP>));
+        else u = ld4(invd_t + c0) * rr;
         st4(rt + c0, rr);
         st4(ut + c0, u);
         v[0] += dot4(rr, u);
@@ -317,8 +426,9 @@ __global__ __launch_bounds__(RBS) void k_mean(HexGeom g, LD X, double* __restric
 //   may equal bsrc).  OF: partial sum |r| -> L1 set 0 and, with of_nf (first residual of a
 //   solve), the normalisation terms -> NF with xref = mean from the k_mean partials.
 // QUAD (nx % 4 == 0, correction absent or sigma_xy only): four cells per lane.
-template <class TP, bool OF, bool QUAD>
-__global__ __launch_bounds__(RBS) void k_residual(HexGeom g, HexOp<double> A,
+// rr0_slot, l1_slot: where the sums of r^2 and |r| go.
+template <class TP, bool OF, bool QUAD, bool LAY>
+__global__ __launch_bounds__(RBS) void k_residual(HexGeom g, HexOp<double> A, Layers<double> L,
                                                   const TP* __restrict__ invd_t,
                                                   const double* __restrict__ xin,
                                                   const double* __restrict__ vcor,
@@ -329,13 +439,14 @@ __global__ __launch_bounds__(RBS) void k_residual(HexGeom g, HexOp<double> A,
                                                   const double* __restrict__ od, unsigned od_mask,
                                                   TP* __restrict__ rt, TP* __restrict__ ut,
                                                   double* __restrict__ part, DevState* S,
-                                                  long long gen, int of_nf)
+                                                  long long gen, int of_nf, int rr0_slot,
+                                                  int l1_slot)
 {
     const bool add_e = e != nullptr && S->outer_gen != gen - 1;
     double xref = 0.0;
     if (OF && of_nf) {
         double xs[1];
-        sum_slots<1>(part, {P_XS}, xs);
+        sum_slots<1>(part, {P_XS}, xs, gridDim.x);
         xref = xs[0] / double((int64_t)g.nx * g.ny * g.nz);
     }
     double v[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
@@ -345,8 +456,8 @@ __global__ __launch_bounds__(RBS) void k_residual(HexGeom g, HexOp<double> A,
     const uint32_t bid = xcd_block(blockIdx.x, gridDim.x);
     if constexpr (QUAD) {
 #define CG_RESIDUAL(LD, XL, CORR)                                                          \
-    residual_range_q<TP, LD, CORR, OF>(g, A, invd_t, XL, vc, xout, bsrc, bout, od, rt, ut,   \
-                                       xref, v, bid)
+    residual_range_q<TP, LD, CORR, OF, LAY>(g, A, L, invd_t, XL, vc, xout, bsrc, bout,       \
+                                            LAY ? L.od : od, rt, ut, xref, v, bid)
         if (od && xprev) CG_RESIDUAL(ExtrapLoad, XE, true);
         else if (od) CG_RESIDUAL(PlainLoad<double>, X0, true);
         else if (xprev) CG_RESIDUAL(ExtrapLoad, XE, false);
@@ -355,8 +466,8 @@ __global__ __launch_bounds__(RBS) void k_residual(HexGeom g, HexOp<double> A,
 #undef CG_RESIDUAL
     } else {
 #define CG_RESIDUAL(LD, XL, CORR)                                                          \
-    residual_range<TP, LD, CORR, OF>(g, A, invd_t, XL, vc, xout, bsrc, bout, od, od_mask,  \
-                                     rt, ut, xref, v)
+    residual_range<TP, LD, CORR, OF, LAY>(g, A, L, invd_t, XL, vc, xout, bsrc, bout, od,     \
+                                          od_mask, rt, ut, xref, v)
         if (od && xprev) CG_RESIDUAL(ExtrapLoad, XE, true);
         else if (od) CG_RESIDUAL(PlainLoad<double>, X0, true);
         else if (xprev) CG_RESIDUAL(ExtrapLoad, XE, false);
@@ -368,10 +479,10 @@ __global__ __launch_bounds__(RBS) void k_residual(HexGeom g, HexOp<double> A,
     if (threadIdx.x == 0) {
         part[(P_G + 0) * RG + bid] = v[0];
         part[(P_RR + 0) * RG + bid] = v[1];
-        part[P_RR0 * RG + bid] = v[2];
+        part[rr0_slot * RG + bid] = v[2];
         part[P_BB * RG + bid] = v[3];
         if (OF) {
-            part[(P_L1 + 0) * RG + bid] = v[4];
+            part[l1_slot * RG + bid] = v[4];
             if (of_nf) part[P_NF * RG + bid] = v[5];
         }
         if (blockIdx.x == 0) {
@@ -416,11 +527,11 @@ __global__ __launch_bounds__(RBS) void k_cg_s(HexGeom g, HexOp<T> A, const T* __
     double rr, rr0, bb, l1 = 0.0, nf = 1.0;
     if (NORM == 1 || (NORM == 2 && k == 0)) {
         double v5[5];
-        sum_slots<5>(part, {P_RR + (k & 1), P_RR0, P_BB, P_L1 + (k & 1), P_NF}, v5);
+        sum_slots<5>(part, {P_RR + (k & 1), P_RR0, P_BB, P_L1 + (k & 1), P_NF}, v5, gridDim.x);
         rr = v5[0]; rr0 = v5[1]; bb = v5[2]; l1 = v5[3]; nf = v5[4] + 1e-20;
     } else {
         double v3[3];
-        sum_slots<3>(part, {P_RR + (k & 1), P_RR0, P_BB}, v3);
+        sum_slots<3>(part, {P_RR + (k & 1), P_RR0, P_BB}, v3, gridDim.x);
         rr = v3[0]; rr0 = v3[1]; bb = v3[2];
     }
     bool outer, conv;
@@ -499,7 +610,7 @@ __global__ __launch_bounds__(RBS) void k_cg_u(HexGeom g, const T* __restrict__ i
 {
     if (S->done_gen == gen) return;
     double v2[2];
-    sum_slots<2>(part, {P_G + (k & 1), P_D}, v2);
+    sum_slots<2>(part, {P_G + (k & 1), P_D}, v2, gridDim.x);
     const double gam = v2[0], del = v2[1];
     double alpha, beta = 0.0;
     if (k == 0) {
@@ -572,6 +683,124 @@ __global__ __launch_bounds__(RBS) void k_cg_u(HexGeom g, const T* __restrict__ i
     }
 }
 
+// ---- Chebyshev's iteration (Golub and Varga, Numer. Math. 3, 1961) with the Jacobi
+// preconditioner.  The rows of D^-1 A differ from the identity by at most
+//   rho = max_i sum_f a_f / (mass + sum_f a_f)
+// in absolute sum, so its spectrum lies in [1 - rho, 1 + rho] with rho known on the host:
+//   z_k = D^-1 (b - A x_k),  x_{k+1} = x_{k-1} + w_{k+1} (x_k - x_{k-1} + z_k),
+//   w_1 = 1, w_2 = 1 / (1 - rho^2 / 2), w_{k+1} = 1 / (1 - rho^2 w_k / 4),
+// after k steps the error (in the norm of D) is at most 2 sigma^k / (1 + sigma^2k) of the
+// first, sigma = rho / (1 + sqrt(1 - rho^2)).  No step needs a dot product, so an iteration
+// is one kernel that reads x_k, x_{k-1}, b and the face coefficients and writes x_{k+1}
+// over x_{k-1}: 16 B per cell FP32 (layered) where the two CG kernels move 56 B and wait
+// for a grid-wide sum each.  At 2.1M cells (rho 0.13) a step takes 7.3 us FP32 and 13.1 us
+// FP64 where a CG iteration took 20.8 and 41.7 us, and the mixed solve's residual passes
+// 22 us with layered coefficients instead of 34 us.
+//
+// One step of x (k_cheb): out = xm + omega (x - xm + (b - A x)/diag), xm null: 0 (the first
+// step, w_1 = 1, needs none).  out may be xm itself.
+//   CORR (first step of a solve, FP64): b += tensor correction of vcor, written back.
+//   NORMS: partial sums |b - A x|^2 -> slot rr_slot, |b|^2 -> P_BB.
+template <class T, bool QUAD, bool LAY, bool CORR, bool NORMS>
+__global__ __launch_bounds__(RBS) void k_cheb(HexGeom g, HexOp<T> A, Layers<T> L, T omega,
+                                              const T* __restrict__ x, const T* xm, T* out,
+                                              T* b, const double* __restrict__ vcor,
+                                              const double* __restrict__ od, unsigned od_mask,
+                                              double* __restrict__ part, int rr_slot)
+{
+    double v[2] = {0.0, 0.0};
+    const uint32_t bid = xcd_block(blockIdx.x, gridDim.x);
+    const PlainLoad<T> X{x};
+    if constexpr (QUAD) {
+        RANGE_LOOP_Q(g)
+        {
+            const int64_t c0 = qi * 4;
+            const IJK q = ijk_of((uint32_t)c0, g);
+            V4<T> bc = ld4(b + c0), xc, d;
+            const V4<T> xo = xm ? ld4(xm + c0) : V4<T>(T(0));
+            if constexpr (CORR) {
+                bc += quad_correction_xy<LAY>(vcor, LAY ? L.od : od, c0, q, g);
+                st4(b + c0, bc);
+            }
+            const V4<T> r = bc - apply_quad_diag<T, LAY>(A, L, X, c0, q, g, xc, d);
+            st4(out + c0, xo + omega * ((xc - xo) + jacobi4<T>(r, d)));
+            if constexpr (NORMS) {
+                v[0] += dot4(r, r);
+                v[1] += dot4(bc, bc);
+            }
+        }
+    } else {
+        RANGE_LOOP_B(g)
+        {
+            const IJK q = ijk_of((uint32_t)c, g);
+            T bc = b[c], xc, d;
+            const T xo = xm ? xm[c] : T(0);
+            if constexpr (CORR) {
+                bc += hex_tensor_correction(vcor, od, n, c, q.i, q.j, q.k, g, od_mask);
+                b[c] = bc;
+            }
+            const T r = bc - apply_row_diag<T, LAY>(A, L, X, c, q, g, xc, d);
+            out[c] = xo + omega * ((xc - xo) + jacobi(r, d));
+            if constexpr (NORMS) {
+                v[0] += double(r) * double(r);
+                v[1] += double(bc) * double(bc);
+            }
+        }
+    }
+    if constexpr (NORMS) {
+        block_sum<RBS, 2>(v);
+        if (threadIdx.x == 0) {
+            part[rr_slot * RG + bid] = v[0];
+            part[P_BB * RG + bid] = v[1];
+        }
+    }
+}
+
+// ---- end of a Chebyshev pass (one block): sums the residual's partials, records whether
+// the step tolerance is met (done_gen/conv_gen, and outer_gen for the refinement) and
+// publishes the state to the host mirror.  rr_slot, l1_slot: the residual tested;
+// init_rr, init_l1 >= 0: slots of the solve's first residual, whose norm becomes init_res.
+//   norm 0: (r,r) <= tol^2 (b,b);  norm 1: sum|r| < tol nf.
+// One thread per partial: at 2.1M cells (1024 partials, 3 slots) the pass ends 6 us sooner
+// than with a block of 256 that sums every slot whether it is asked for or not.
+__global__ __launch_bounds__(RG) void k_cheb_check(const double* __restrict__ part, int nb,
+                                                   DevState* S, DevState* pub, long long gen,
+                                                   int norm, double tol, int rr_slot,
+                                                   int l1_slot, int init_rr, int init_l1)
+{
+    // the slots this norm needs: residual, its scale, the solve's first residual
+    const int sl[3] = {norm ? l1_slot : rr_slot, norm ? (int)P_NF : (int)P_BB,
+                       norm ? init_l1 : init_rr};
+    double v[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+        v[k] = sl[k] >= 0 && (int)threadIdx.x < nb ? part[sl[k] * RG + threadIdx.x] : 0.0;
+    block_sum<RG, 3>(v);
+    if (threadIdx.x == 0) {
+        const double nf = v[1] + 1e-20;
+        const bool conv = norm ? v[0] < tol * nf : v[0] <= tol * tol * v[1];
+        if (norm) {
+            S->nf = nf;
+            S->l1_0 = S->l1 = v[0];
+        } else {
+            S->s[S_R0] = S->s[S_RR] = v[0];
+            S->s[S_BB] = v[1];
+        }
+        if (sl[2] >= 0)
+            S->init_res = norm ? v[2] / nf : sqrt(v[2] / (v[1] > 0.0 ? v[1] : 1.0));
+        S->iters = 0;      // the host knows a Chebyshev pass's steps
+        if (conv) {
+            S->outer_gen = gen;
+            S->conv_gen = gen;
+            S->done_gen = gen;
+        }
+    }
+    __syncthreads();   // thread 0's updates of S before the copy by the block's lanes
+    if (threadIdx.x < sizeof(DevState) / 8)
+        reinterpret_cast<volatile unsigned long long*>(pub)[threadIdx.x] =
+            reinterpret_cast<const volatile unsigned long long*>(S)[threadIdx.x];
+}
+
 // ---- activation time (myocardiumDomain.C:345-374) and V^{n+1} = x when x is elsewhere;
 // with a gate it runs only when the solve of that generation met the step tolerance
 __global__ __launch_bounds__(BS) void k_activation(HexGeom g, const double* __restrict__ Vn,
@@ -632,7 +861,7 @@ const char* kernel_name(int id)
 {
     static const char* names[K_COUNT] = {"ionic",    "spmv_dot",   "cg_update", "residual_first",
                                          "residual", "activation", "invdiag",    "apply",
-                                         "pseudo_ecg"};
+                                         "pseudo_ecg", "chebyshev"};
     return id >= 0 && id < K_COUNT ? names[id] : "?";
 }
 
@@ -678,6 +907,17 @@ struct ImplicitSolver {
                                      // writes S there, so no copy kernel runs
     hipEvent_t read_done = nullptr;  // after the kernel that published S
     double mass_c = -1.0;    // coefft of the current invd
+    unsigned rgrid = RG;     // blocks of the reducing kernels
+    bool layered = false;    // conductivity constant in each z-plane: coefficients from lay
+    double *lay = nullptr, *lay_od = nullptr;  // [nz][3] fx, fy, fz; [nz] sigma_xy
+    float* lay32 = nullptr;
+    double smax = 0.0;       // largest sum of a row's face coefficients
+    // Chebyshev: initial residuals of the last step's correctors (in the controls' norm; 0:
+    // unknown) that size the next step's iteration, and whether x0 of the next FP64 solve
+    // was written into V^{n+1} (else into xalt)
+    double last_init_res[4] = {0.0, 0.0, 0.0, 0.0};
+    bool x0_in_new = false;
+    bool next_even = false;
     bool quad = false;       // nx % 4 == 0: CG kernels on quads of cells (vector loads)
     long long gen = 0;       // generation of the last CG solve started
     int64_t total_iters = 0;
@@ -694,6 +934,7 @@ int implicit_set_controls(ImplicitSolver* S, const SolveControls& c)
 {
     if (c.norm != 0 && c.norm != 1) return 1;
     S->ctl = c;
+    for (double& r : S->last_init_res) r = 0.0;
     if (c.n_outer > 1 && S->prec == 1 && S->od && !S->bc &&
         hipMalloc((void**)&S->bc, 8 * S->n) != hipSuccess)
         return 5;
@@ -717,6 +958,10 @@ template <> HexOp<float> op_of<float>(const ImplicitSolver* S, double c)
     return {S->fx32, S->fy32, S->fz32, S->invd32, float(c * S->chiCm / S->dt)};
 }
 
+template <class T> static Layers<T> layers_of(const ImplicitSolver* S);
+template <> Layers<double> layers_of<double>(const ImplicitSolver* S) { return {S->lay, S->lay_od}; }
+template <> Layers<float> layers_of<float>(const ImplicitSolver* S) { return {S->lay32, nullptr}; }
+
 int implicit_create(ImplicitSolver** out, const HexGeom& g, const double* sig, double chiCm,
                     double dt, int prec, hipStream_t s, std::string* err)
 {
@@ -727,18 +972,32 @@ int implicit_create(ImplicitSolver** out, const HexGeom& g, const double* sig, d
     const int64_t n = S->n;
     const int64_t sy = g.nx, sz = (int64_t)g.nx * g.ny;
     std::vector<double> fx(n, 0.0), fy(n, 0.0), fz(n, 0.0), od(3 * n, 0.0);
-    for (int64_t c = 0; c < n; ++c) {
-        const int i = (int)(c % g.nx), j = (int)((c / g.nx) % g.ny), k = (int)(c / sz);
-        if (i < g.nx - 1) fx[c] = 0.5 * (sig[9 * c + 0] + sig[9 * (c + 1) + 0]) / (g.hx * g.hx);
-        if (j < g.ny - 1) fy[c] = 0.5 * (sig[9 * c + 4] + sig[9 * (c + sy) + 4]) / (g.hy * g.hy);
-        if (k < g.nz - 1) fz[c] = 0.5 * (sig[9 * c + 8] + sig[9 * (c + sz) + 8]) / (g.hz * g.hz);
-        od[c] = sig[9 * c + 1];
-        od[n + c] = sig[9 * c + 2];
-        od[2 * n + c] = sig[9 * c + 5];
-        for (int q = 0; q < 3; ++q)
-            if (od[q * n + c] != 0.0) S->od_mask |= 1u << q;
+    S->layered = true;
+    int64_t c = 0;
+    for (int k = 0; k < g.nz; ++k) {
+        const double* p = sig + 9 * c;   // the plane's first cell
+        for (int j = 0; j < g.ny; ++j)
+            for (int i = 0; i < g.nx; ++i, ++c) {
+                const double* t = sig + 9 * c;
+                if (i < g.nx - 1) fx[c] = 0.5 * (t[0] + t[9]) / (g.hx * g.hx);
+                if (j < g.ny - 1) fy[c] = 0.5 * (t[4] + t[9 * sy + 4]) / (g.hy * g.hy);
+                if (k < g.nz - 1) fz[c] = 0.5 * (t[8] + t[9 * sz + 8]) / (g.hz * g.hz);
+                od[c] = t[1];
+                od[n + c] = t[2];
+                od[2 * n + c] = t[5];
+                S->od_mask |= (t[1] != 0.0 ? 1u : 0u) | (t[2] != 0.0 ? 2u : 0u) |
+                              (t[5] != 0.0 ? 4u : 0u);
+                if (t[0] != p[0] || t[4] != p[4] || t[8] != p[8] || t[1] != p[1])
+                    S->layered = false;
+                const double sum = fx[c] + (i > 0 ? fx[c - 1] : 0.0) + fy[c] +
+                                   (j > 0 ? fy[c - sy] : 0.0) + fz[c] + (k > 0 ? fz[c - sz] : 0.0);
+                // (a NaN, or a negative coefficient, stays as NaN: no Chebyshev)
+                if (fx[c] < 0.0 || fy[c] < 0.0 || fz[c] < 0.0) S->smax = NAN;
+                else if (!(sum <= S->smax) && S->smax == S->smax) S->smax = sum;
+            }
     }
     const bool offdiag = S->od_mask != 0;
+    S->rgrid = reduce_grid(S->quad ? n / 4 : n);
     bool ok = true;
     auto A = [&](void** ptr, size_t bytes) { ok &= hipMalloc(ptr, bytes) == hipSuccess; };
     A((void**)&S->fx, 8 * n); A((void**)&S->fy, 8 * n); A((void**)&S->fz, 8 * n);
@@ -747,13 +1006,17 @@ int implicit_create(ImplicitSolver** out, const HexGeom& g, const double* sig, d
     A((void**)&S->partials, 8 * RG * P_NSLOT);
     A((void**)&S->S, sizeof(DevState));
     if (offdiag) A((void**)&S->od, 8 * 3 * n);
+    A((void**)&S->xalt, 8 * n);
+    if (S->layered) {
+        A((void**)&S->lay, 8 * 3 * g.nz); A((void**)&S->lay_od, 8 * g.nz);
+        A((void**)&S->lay32, 4 * 3 * g.nz);
+    }
     if (prec == 1) {
         A((void**)&S->fx32, 4 * n); A((void**)&S->fy32, 4 * n); A((void**)&S->fz32, 4 * n);
         A((void**)&S->invd32, 4 * n);
         A((void**)&S->v32.r, 4 * n); A((void**)&S->v32.u, 4 * n); A((void**)&S->v32.p, 4 * n);
         A((void**)&S->v32.s, 4 * n); A((void**)&S->v32.w, 4 * n);
         A((void**)&S->e32, 4 * n);
-        A((void**)&S->xalt, 8 * n);
     } else {
         A((void**)&S->v64.r, 8 * n); A((void**)&S->v64.u, 8 * n); A((void**)&S->v64.p, 8 * n);
         A((void**)&S->v64.s, 8 * n); A((void**)&S->v64.w, 8 * n);
@@ -780,6 +1043,20 @@ int implicit_create(ImplicitSolver** out, const HexGeom& g, const double* sig, d
         for (int64_t c = 0; c < n; ++c) f[c] = (float)fz[c];
         hipMemcpy(S->fz32, f.data(), 4 * n, hipMemcpyHostToDevice);
     }
+    if (S->layered) {
+        std::vector<double> l(3 * g.nz), lo(g.nz);
+        for (int k = 0; k < g.nz; ++k) {
+            // the faces of the plane's first cell; 0 where the block is one cell thick
+            l[3 * k] = fx[k * sz];
+            l[3 * k + 1] = fy[k * sz];
+            l[3 * k + 2] = fz[k * sz];
+            lo[k] = od[k * sz];
+        }
+        std::vector<float> l32(l.begin(), l.end());
+        hipMemcpy(S->lay, l.data(), 8 * l.size(), hipMemcpyHostToDevice);
+        hipMemcpy(S->lay_od, lo.data(), 8 * lo.size(), hipMemcpyHostToDevice);
+        hipMemcpy(S->lay32, l32.data(), 4 * l32.size(), hipMemcpyHostToDevice);
+    }
     DevState z{};
     z.done_gen = -1;
     z.outer_gen = -1;
@@ -792,7 +1069,8 @@ int implicit_create(ImplicitSolver** out, const HexGeom& g, const double* sig, d
 void implicit_destroy(ImplicitSolver* S)
 {
     if (!S) return;
-    void* ptrs[] = {S->bc,     S->fx,     S->fy,     S->fz,     S->invd,     S->b,        S->xalt,
+    void* ptrs[] = {S->lay,    S->lay_od, S->lay32,
+                    S->bc,     S->fx,     S->fy,     S->fz,     S->invd,     S->b,        S->xalt,
                     S->partials, S->S,    S->od,     S->fx32,     S->fy32,     S->fz32,
                     S->invd32, S->v32.r,  S->v32.u,  S->v32.p,    S->v32.s,    S->v32.w,
                     S->e32,    S->v64.r,  S->v64.u,  S->v64.p,    S->v64.s,    S->v64.w};
@@ -865,7 +1143,7 @@ template <class T> struct CgRun {
         const double of_rel = S->ctl.rel_tol;
         DevState* pub = publish ? S->hS_dev : nullptr;
 #define CG_S(Q, N)                                                                         \
-    hipLaunchKernelGGL((k_cg_s<T, Q, N>), dim3(RG), dim3(RBS), 0, S->stream, S->g, A,      \
+    hipLaunchKernelGGL((k_cg_s<T, Q, N>), dim3(S->rgrid), dim3(RBS), 0, S->stream, S->g, A,      \
                        (const T*)v.u, v.w, S->partials, S->S, gen, k, tol2, rel, abs2,     \
                        outer_tol2, max_iter, of_tol, of_rel, record_init, pub)
         switch (norm_kind() + (S->quad ? 3 : 0)) {
@@ -887,7 +1165,7 @@ template <class T> struct CgRun {
         const int tk = prof ? prof->begin(K_UPDATE) : -1;
         const bool l1 = norm_kind() == 1;
 #define CG_U(Q, L)                                                                         \
-    hipLaunchKernelGGL((k_cg_u<T, TX, Q, L>), dim3(RG), dim3(RBS), 0, S->stream, S->g,     \
+    hipLaunchKernelGGL((k_cg_u<T, TX, Q, L>), dim3(S->rgrid), dim3(RBS), 0, S->stream, S->g,     \
                        A.invd, x, v.r, v.u, v.p, v.s, (const T*)v.w, S->partials, S->S,    \
                        gen, k, x_from_zero)
         if (S->quad) {
@@ -907,35 +1185,85 @@ template <class T> struct CgRun {
     void mean(const double* xin, const double* xprev)
     {
         if (xprev)
-            hipLaunchKernelGGL((k_mean<ExtrapLoad>), dim3(RG), dim3(RBS), 0, S->stream, S->g,
+            hipLaunchKernelGGL((k_mean<ExtrapLoad>), dim3(S->rgrid), dim3(RBS), 0, S->stream, S->g,
                                ExtrapLoad{xin, xprev}, S->partials);
         else
-            hipLaunchKernelGGL((k_mean<PlainLoad<double>>), dim3(RG), dim3(RBS), 0, S->stream,
+            hipLaunchKernelGGL((k_mean<PlainLoad<double>>), dim3(S->rgrid), dim3(RBS), 0, S->stream,
                                S->g, PlainLoad<double>{xin}, S->partials);
     }
     void residual(int kid, long long gen, const double* xin, const double* xprev,
                   const float* e, double* xout, const double* od, const HexOp<double>& A64,
-                  const double* bsrc, double* bout, int of_nf, const double* vcor = nullptr)
+                  const double* bsrc, double* bout, int of_nf, const double* vcor = nullptr,
+                  int rr0_slot = P_RR0, int l1_slot = P_L1)
     {
         const int tk = prof ? prof->begin(kid) : -1;
         // quads need nx % 4 == 0 and no correction beyond sigma_xy
         const bool quad = S->quad && (!od || S->od_mask == 1u);
-#define CG_R(OF, Q, NF)                                                                    \
-    hipLaunchKernelGGL((k_residual<T, OF, Q>), dim3(RG), dim3(RBS), 0, S->stream, S->g, A64, \
-                       (const T*)A.invd, xin, vcor, xprev, e, xout, bsrc, bout, od, S->od_mask, \
-                       v.r,                                                                \
-                       v.u, S->partials, S->S, gen, NF)
+        const Layers<double> L = layers_of<double>(S);
+#define CG_R(OF, Q, LAY, NF)                                                               \
+    hipLaunchKernelGGL((k_residual<T, OF, Q, LAY>), dim3(S->rgrid), dim3(RBS), 0, S->stream, \
+                       S->g, A64, L, (const T*)A.invd, xin, vcor, xprev, e, xout, bsrc,     \
+                       bout, od, S->od_mask, v.r, v.u, S->partials, S->S, gen, NF, rr0_slot, \
+                       l1_slot)
+#define CG_RL(OF, Q, NF)                                                                   \
+    do {                                                                                   \
+        if (S->layered) CG_R(OF, Q, true, NF);                                             \
+        else CG_R(OF, Q, false, NF);                                                       \
+    } while (0)
         if (S->ctl.norm == 1) {
-            if (quad) CG_R(true, true, of_nf);
-            else CG_R(true, false, of_nf);
+            if (quad) CG_RL(true, true, of_nf);
+            else CG_RL(true, false, of_nf);
         } else {
-            if (quad) CG_R(false, true, 0);
-            else CG_R(false, false, 0);
+            if (quad) CG_RL(false, true, 0);
+            else CG_RL(false, false, 0);
         }
+#undef CG_RL
 #undef CG_R
         if (prof) prof->end(tk);
     }
 };
+
+// one Chebyshev step out = xm + omega (x - xm + D^-1 (b - A x)); corr: b += correction of
+// vcor first; rr_slot >= 0: with the residual's partial sums
+template <class T>
+void cheb_step(ImplicitSolver* S, Profiler* prof, const HexOp<T>& A, double omega, const T* x,
+               const T* xm, T* out, T* b, const double* vcor, bool corr, int rr_slot)
+{
+    const int tk = prof ? prof->begin(K_CHEB) : -1;
+    // quads need nx % 4 == 0 and no correction beyond sigma_xy
+    const bool quad = S->quad && (!corr || S->od_mask == 1u);
+    const Layers<T> L = layers_of<T>(S);
+#define CG_C(Q, LAY, CO, NO)                                                               \
+    hipLaunchKernelGGL((k_cheb<T, Q, LAY, CO, NO>), dim3(S->rgrid), dim3(RBS), 0, S->stream, \
+                       S->g, A, L, T(omega), x, xm, out, b, vcor, (const double*)S->od,    \
+                       S->od_mask, S->partials, rr_slot)
+#define CG_CQ(CO, NO)                                                                      \
+    do {                                                                                   \
+        if (quad && S->layered) CG_C(true, true, CO, NO);                                  \
+        else if (quad) CG_C(true, false, CO, NO);                                          \
+        else if (S->layered) CG_C(false, true, CO, NO);                                    \
+        else CG_C(false, false, CO, NO);                                                   \
+    } while (0)
+    if constexpr (sizeof(T) == 8) {
+        if (corr) CG_CQ(true, true);
+        else if (rr_slot >= 0) CG_CQ(false, true);
+        else CG_CQ(false, false);
+    } else {
+        CG_CQ(false, false);
+    }
+#undef CG_CQ
+#undef CG_C
+    if (prof) prof->end(tk);
+}
+
+// steps k of Chebyshev's iteration whose bound 2 sigma^k / (1 + sigma^2k) is at most need
+int cheb_steps(double rho, double need)
+{
+    const double sg = rho / (1.0 + std::sqrt(1.0 - rho * rho));
+    int k = 1;
+    for (double p = sg; 2.0 * p / (1.0 + p * p) > need && k < 64; ++k) p *= sg;
+    return k;
+}
 
 // drop the timing records of launches of solve `gen` beyond its `iters` iterations
 // (S-kernels with k >= iters only tested convergence, U-kernels with k >= iters did nothing)
@@ -962,11 +1290,27 @@ int implicit_step(ImplicitSolver* S, int model, int prec, int tissue, void* stat
     // Outer correctors keep the extrapolation in the residual.
     const bool fuse = S->ctl.n_outer <= 1;
     const double* od_res = S->od;
-    const bool x0_fused = fuse && prec == 1 && extrapolate;
+    // Chebyshev's iteration where rho <= 0.6: there it needs at most about one step in four
+    // more than the conjugate gradients (whose count the bound also limits), each a third of
+    // their time, and one Jacobi step never enlarges a residual (rho sqrt(dmax/dmin) < 1 as
+    // dmax/dmin <= 1/(1 - rho)).  Not for OpenFOAM's norm in FP64, whose solves the PIMPLE
+    // loop counts, nor for tolerances at the rounding of the true residual it tests, nor
+    // when few iterations are allowed, nor in FP64 up to SMALL_N cells, where a solve is
+    // launches and waits whichever iteration it runs.
+    auto rho_of = [&](double c) { return S->smax / (c * S->chiCm / S->dt + S->smax); };
+    auto use_cheb = [&](double c) {
+        return rho_of(c) <= 0.6 && max_iter >= 100 &&
+               (prec == 1 || (S->ctl.norm == 0 && fuse && tol >= 1e-13 && S->n > SMALL_N));
+    };
+    const double rho = rho_of(st.c);
+    const bool cheb = use_cheb(st.c);
+    const bool x0_fused = fuse && extrapolate && (prec == 1 || cheb);
     if (!ionic_queued) {
+        S->x0_in_new = prec == 0 && S->next_even;
         tk = prof ? prof->begin(K_IONIC) : -1;
         e = launch_ionic_rhs(model, prec, tissue, S->g, states, Vn, Vm1,
-                             x0_fused ? S->xalt : nullptr, Iion, S->b, st, P, S->stream);
+                             x0_fused ? (S->x0_in_new ? Vnew : S->xalt) : nullptr, Iion, S->b,
+                             st, P, S->stream);
         if (prof) prof->end(tk);
         if (e != hipSuccess) { *err = std::string("ionic/rhs launch: ") + hipGetErrorString(e); return 4; }
     }
@@ -1020,9 +1364,12 @@ int implicit_step(ImplicitSolver* S, int model, int prec, int tissue, void* stat
                 sn.act_v = st.act_v;
             }
             int t = prof ? prof->begin(K_IONIC) : -1;
-            launch_ionic_rhs(model, prec, tissue, S->g, states, Vnew, Vn,
-                             fuse && prec == 1 ? S->xalt : nullptr, Iion, S->b, sn, P,
-                             S->stream);
+            // (the next step's V^{n+1} is this one's V^{n-1}, whose last reader is done)
+            S->x0_in_new = prec == 0 && S->next_even;
+            double* x0 = !fuse || !(prec == 1 || use_cheb(sn.c)) ? nullptr
+                         : S->x0_in_new ? const_cast<double*>(Vm1) : S->xalt;
+            launch_ionic_rhs(model, prec, tissue, S->g, states, Vnew, Vn, x0, Iion, S->b, sn,
+                             P, S->stream);
             if (prof) prof->end(t);
         }
         if (hipGetLastError() != hipSuccess) return false;
@@ -1035,16 +1382,76 @@ int implicit_step(ImplicitSolver* S, int model, int prec, int tissue, void* stat
     double prev_init = 0.0;
     int solves = 0;
     if (prec == 0) {
-        // fp64 CG per corrector; x0 = V^n (copied into V^{n+1} by the first residual)
         CgRun<double> cg{S, A, S->v64, prof, &log};
+        // Chebyshev from x0 = 2 V^n - V^{n-1} (V^n on the first step): a Jacobi step from x0,
+        // the iteration, a last Jacobi step whose kernel tests the residual of the iterate
+        // before it.  A pass that misses the tolerance is repeated from its result, with the
+        // steps its own residual asks for; after three the conjugate gradients take over.
+        bool started = false;      // V^{n+1} holds an iterate, b the correction
+        for (int pass = 0; cheb && pass < 3; ++pass) {
+            const long long gen = ++S->gen;
+            const double r0 = pass == 0 ? S->last_init_res[0] : S->last_res;
+            double need = r0 > 0.0 ? 0.5 * tol / r0 : 1e-5;
+            need = need < 0.3 ? need : 0.3;
+            int J = cheb_steps(rho, need) + 1;
+            const double* x = pass > 0 ? Vnew : x0_fused ? (S->x0_in_new ? Vnew : S->xalt) : Vn;
+            // x_J lands in V^{n+1}
+            if (x == Vnew) J += J & 1;
+            else if (x == S->xalt) J += !(J & 1);
+            const double* xm = nullptr;
+            double w = 1.0;
+            for (int j = 0; j < J; ++j) {
+                double* out = ((J - j) & 1) ? Vnew : S->xalt;
+                const bool ends = j == 0 || j == J - 1;
+                if (j == 1) w = 1.0 / (1.0 - 0.5 * rho * rho);
+                else if (j > 1) w = 1.0 / (1.0 - 0.25 * rho * rho * w);
+                cheb_step<double>(S, prof, A, ends ? 1.0 : w, x, ends ? nullptr : xm, out, S->b,
+                                  Vn, j == 0 && pass == 0 && od_res,
+                                  j == 0 ? P_RRI : j == J - 1 ? P_RR0 : -1);
+                xm = x;
+                x = out;
+            }
+            started = true;
+            S->next_even = !(J & 1);
+            hipLaunchKernelGGL(k_cheb_check, dim3(1), dim3(RG), 0, S->stream,
+                               (const double*)S->partials, (int)S->rgrid, S->S, S->hS_dev, gen,
+                               0, tol, P_RR0, P_RR0, pass == 0 ? P_RRI : -1, -1);
+            size_t gated;
+            if (!finish_and_read(gen, Vnew, &gated, true)) {
+                *err = "Chebyshev launch or read-back failed";
+                return 4;
+            }
+            const DevState& h = *S->hS;
+            const bool ok = h.conv_gen == gen;
+            if (prof) {
+                if (!ok) prof->invalidate_range(gated, prof->mark());
+                prof->resolve(false);
+            }
+            used_total += J;
+            S->last_res = std::sqrt(h.s[S_RR] / (h.s[S_BB] > 0 ? h.s[S_BB] : 1.0));
+            if (pass == 0) {
+                prev_init = h.init_res;
+                S->last_init_res[0] = prev_init;
+            }
+            if (ok) {
+                S->last_solves = 1;
+                S->last_init = prev_init;
+                S->last_final = S->last_res;
+                S->total_iters += used_total;
+                return 0;
+            }
+            if (!std::isfinite(S->last_res)) break;
+        }
+        // fp64 CG per corrector; x0 = V^n (copied into V^{n+1} by the first residual)
         for (int outer = 1;; ++outer) {
             const bool last = n_outer == 1 || outer >= n_outer ||
                               (outer > 1 && prev_init < S->ctl.residual_control);
             const long long gen = ++S->gen;
-            const double* xin = outer == 1 ? Vn : Vnew;
+            const bool from_vn = outer == 1 && !started;
+            const double* xin = from_vn ? Vn : Vnew;
             if (of) cg.mean(xin, nullptr);
-            cg.residual(K_RESIDUAL0, gen, xin, nullptr, nullptr, outer == 1 ? Vnew : nullptr,
-                        outer == 1 ? od_res : S->od, A, S->b, nullptr, 1);
+            cg.residual(K_RESIDUAL0, gen, xin, nullptr, nullptr, from_vn ? Vnew : nullptr,
+                        started ? nullptr : S->od, A, S->b, nullptr, 1);
             cg.s_kernel(gen, 0, tol * tol, 0, 0.0, 0.0, max_iter, tol, 1);
             int k = 0;
             int chunk = S->last_inner + 1 > 2 ? S->last_inner + 1 : 2;
@@ -1072,6 +1479,7 @@ int implicit_step(ImplicitSolver* S, int model, int prec, int tissue, void* stat
                     const double bb = h.s[S_BB] > 0 ? h.s[S_BB] : 1.0;
                     S->last_res = of ? h.l1 / h.nf : std::sqrt(h.s[S_RR] / bb);
                     prev_init = h.init_res;
+                    if (S->last_init_res[0] == 0.0) S->last_init_res[0] = prev_init;
                     if (!ok) {
                         *err = "PCG did not converge within max_iter";
                         return 7;
@@ -1099,32 +1507,92 @@ int implicit_step(ImplicitSolver* S, int model, int prec, int tissue, void* stat
         double* bcur = od_res ? (n_outer > 1 ? S->bc : S->b) : nullptr;
         const double* bref = bcur ? bcur : S->b;
         const double* cur = Vn;
+        float* const eb[2] = {S->v32.u, S->v32.p};
+        int ei = 0;   // eb[ei]: M^-1 r of the last residual, the first Chebyshev iterate
         for (int outer = 1;; ++outer) {
             const bool last = n_outer == 1 || outer >= n_outer ||
                               (outer > 1 && prev_init < S->ctl.residual_control);
             long long gen = ++S->gen;
+            // a Chebyshev pass keeps the corrector's first residual in slots of its own
+            const int rr_i = cheb ? P_RRI : P_RR0, l1_i = cheb ? P_L1 + 1 : P_L1;
             if (outer == 1 && x0_fused) {
                 // x0 = 2 V^n - V^{n-1} already in xalt (ionic kernel), so the first
                 // refinement lands in V^{n+1} itself
                 if (of) cg.mean(S->xalt, nullptr);
                 cg.residual(K_RESIDUAL0, gen, S->xalt, nullptr, nullptr, nullptr, od_res, A,
-                            S->b, bcur, 1, Vn);
+                            S->b, bcur, 1, Vn, rr_i, l1_i);
                 cur = S->xalt;
             } else if (outer == 1) {
                 // x0 = 2 V^n - V^{n-1} (V^n on the first step), written to xalt
                 const double* xprev = extrapolate ? Vm1 : nullptr;
                 if (of) cg.mean(Vn, xprev);
                 cg.residual(K_RESIDUAL0, gen, Vn, xprev, nullptr, xprev ? S->xalt : nullptr,
-                            od_res, A, S->b, bcur, 1);
+                            od_res, A, S->b, bcur, 1, nullptr, rr_i, l1_i);
                 cur = xprev ? S->xalt : Vn;
             } else {
                 if (of) cg.mean(cur, nullptr);
                 cg.residual(K_RESIDUAL0, gen, cur, nullptr, nullptr, nullptr, S->od, A, S->b,
-                            bcur, 1);
+                            bcur, 1, nullptr, rr_i, l1_i);
             }
-            cg.s_kernel(gen, 0, inner_tol * inner_tol, 1, abs2, tol * tol, max_iter, tol, 1);
+            if (!cheb)
+                cg.s_kernel(gen, 0, inner_tol * inner_tol, 1, abs2, tol * tol, max_iter, tol, 1);
             bool init_read = false;
+            double& hist = S->last_init_res[outer < 4 ? outer - 1 : 3];
             for (int pass = 0;; ++pass) {
+                // Chebyshev: correction e of x from e = 0, whose first iterate M^-1 r came with
+                // the residual; as many steps as the last residual (or, in a corrector's first
+                // pass, the last step's initial residual) is above the tolerance, at most
+                // what FP32 resolves
+                if (cheb && pass < 4) {
+                    const double r0 = pass == 0 ? hist : S->last_res;
+                    double need = r0 > 0.0 ? 0.5 * tol / r0 : 1e-5;
+                    need = need < 1e-6 ? 1e-6 : need < 0.3 ? need : 0.3;
+                    const int K = cheb_steps(rho, need);
+                    double w = 1.0;
+                    for (int j = 1; j < K; ++j) {
+                        w = j == 1 ? 1.0 / (1.0 - 0.5 * rho * rho)
+                                   : 1.0 / (1.0 - 0.25 * rho * rho * w);
+                        cheb_step<float>(S, prof, cg.A, w, eb[ei], j == 1 ? nullptr : eb[ei ^ 1],
+                                         eb[ei ^ 1], S->v32.r, nullptr, false, -1);
+                        ei ^= 1;
+                    }
+                    double* nxt = cur == Vnew ? S->xalt : Vnew;
+                    const long long ngen = ++S->gen;
+                    cg.v.u = eb[ei ^ 1];   // the residual reads e in eb[ei] while it writes u
+                    cg.v.p = eb[ei];
+                    cg.residual(K_RESIDUAL, ngen, cur, nullptr, eb[ei], nxt, nullptr, A, bref,
+                                nullptr, 0);
+                    ei ^= 1;
+                    hipLaunchKernelGGL(k_cheb_check, dim3(1), dim3(RG), 0, S->stream,
+                                       (const double*)S->partials, (int)S->rgrid, S->S,
+                                       S->hS_dev, ngen, of ? 1 : 0, tol, P_RR0, P_L1,
+                                       pass == 0 ? rr_i : -1, pass == 0 ? l1_i : -1);
+                    cur = nxt;
+                    size_t gated;
+                    if (!finish_and_read(ngen, cur, &gated, last)) {
+                        *err = "Chebyshev launch or read-back failed";
+                        return 4;
+                    }
+                    const DevState& h = *S->hS;
+                    if (!init_read) {
+                        hist = prev_init = h.init_res;
+                        init_read = true;
+                    }
+                    const bool finished = h.outer_gen == ngen;
+                    if (!finished && prof && last) prof->invalidate_range(gated, prof->mark());
+                    if (prof) prof->resolve(false);
+                    used_total += K;
+                    S->last_res = of ? h.l1 / h.nf
+                                     : std::sqrt(h.s[S_R0] / (h.s[S_BB] > 0 ? h.s[S_BB] : 1.0));
+                    if (finished) break;
+                    gen = ngen;
+                    if (pass == 3) {   // the conjugate gradients take over from this residual
+                        S->iters_sum_seen = h.iters_sum;
+                        cg.s_kernel(gen, 0, inner_tol * inner_tol, 1, abs2, tol * tol, max_iter,
+                                    tol, 0);
+                    }
+                    continue;
+                }
                 const int chunk = S->last_inner + 1 > 2 ? S->last_inner + 1 : 2;
                 for (int k = 0; k < chunk; ++k) {
                     cg.u_kernel(gen, k, S->e32, 1);

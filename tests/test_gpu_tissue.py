@@ -268,3 +268,37 @@ def test_activation_threshold(gpu, orc, algorithm):
              (thr, (a > 0).sum(), np.max(np.abs(a - want))))
         np.testing.assert_array_equal(a > 0, want > 0)
         assert np.max(np.abs(a - want)) <= 1e-12
+
+
+@pytest.mark.parametrize("h", [2e-4, 7e-5, 4e-5])
+@pytest.mark.parametrize("kind", ["layered", "cellwise"])
+@pytest.mark.parametrize("shape", [(16, 8, 6), (13, 7, 5), (8, 1, 1), (4, 5, 1), (1, 1, 9),
+                                   (260, 9, 5), (101, 12, 8)])
+def test_implicit_solver_branches(gpu, orc, shape, kind, h):
+    """Chebyshev's iteration (h = 0.2 and 0.07 mm: rho 0.13 and 0.55) and the conjugate
+    gradients (0.04 mm: rho 0.79), quads and single cells, coefficients per plane and per
+    cell (with all off-diagonal conductivities), one cell thick, on both sides of the 8192
+    cells up to which FP64 stays with the conjugate gradients: the oracle's solution.
+    FP64: both solve to 1e-12 of b, whose error reaches Vm through at most 40 steps; mixed:
+    FP32 gates, 40 steps of a few FP32 roundings each."""
+    _say("solver branches", shape, kind, h)
+    m, tis, key, word, _ = MODELS["BO_epi"]
+    sig = np.asarray(rotating_fibre_sigma(*shape)).reshape(-1, 9).copy()
+    if kind == "cellwise":
+        rng = np.random.default_rng(4)
+        sig *= rng.uniform(0.6, 1.0, (sig.shape[0], 1))
+        for d, e in ((2, 6), (5, 7)):
+            sig[:, d] = sig[:, e] = rng.uniform(-5e-3, 5e-3, sig.shape[0])
+    dt, n_steps = 2e-5, 40
+    box = dict(BOX, stimulusLocationMax=[3 * h, 3 * h, 3 * h], stimulusIntensity=1e6)
+    T = _oracle_run(orc, shape, h, sig, m, tis, dt, n_steps, 0, 1, box, pcg_tol=1e-12)
+    for prec, bound in (("fp64", 1e-9), ("mixed", 2e-5)):
+        dom = gpu.Monodomain(gpu.HexMesh(*shape, h),
+                             _coeffs(key, word, "implicit", sigma=sig, box=box), dt=dt,
+                             tol=1e-12, max_iter=5000, precision=prec)
+        dom.step(n_steps)
+        err = np.max(np.abs(dom.Vm - T.V)) / np.max(np.abs(T.V))
+        iters, res = dom.solver_stats()
+        _say("  %s: Vm rel %.2e, %d iterations, residual %.1e" % (prec, err, iters, res))
+        assert res <= 1e-12 and iters > 0
+        assert err <= bound
