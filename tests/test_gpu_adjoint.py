@@ -301,3 +301,36 @@ def test_implicit_adjoint_gradient_vs_oracle_finite_differences(gpu, orc):
         fd = (fp - fm) / (2 * e[i])
         _say("  theta %d: adjoint %.9e fd %.9e" % (i, gt[i], fd))
         assert abs(gt[i] - fd) <= 1e-5 * abs(fd)
+
+
+@pytest.mark.parametrize("shape,h", [((12, 10, 6), 2e-4), ((9, 1, 1), 2e-4), ((7, 5, 1), 4e-5),
+                                     ((12, 10, 6), 4e-5), ((12, 10, 6), 2e-5)])
+def test_implicit_adjoint_solver_branches(gpu, orc, shape, h):
+    """The fixed-length Chebyshev solves (rho 0.07 at h = 0.2 mm and 0.65 a, 0.04 mm: the
+    PCG above 0.6) against the run's own central difference in a random kappa direction.
+    The potentials stay below the switches' first threshold, so the loss is smooth: the
+    difference carries eps^2 truncation (1e-6 relative at eps 1e-3) and the loss's 1e-15
+    rounding over eps."""
+    import torch
+    _say("implicit adjoint branches", shape, h)
+    mesh, dom = _dom(gpu, shape, h, "implicit", tol=1e-13, box_max=[-1.0, -1.0, -1.0])
+    n, steps = mesh.n, 12
+    rng = np.random.default_rng(3)
+    dom.set_field(0, -0.084 + 4e-4 * rng.random(n))
+    cells = rng.choice(n, min(5, n), replace=False)
+    adj = gpu.TissueAdjoint(dom, cells, checkpoint_every=5)
+    target = torch.tensor(-0.084 + 4e-4 * rng.random((steps, cells.size)), device="cuda")
+    kappa0, d = rng.uniform(0.8, 1.25, n), rng.standard_normal(n)
+    theta = torch.tensor([0.11, 1.8875], dtype=torch.float64)
+
+    def loss(k):
+        return ((gpu.probe_traces(adj, k, theta, steps) - target) ** 2).sum() * 1e6
+
+    kappa = torch.tensor(kappa0, dtype=torch.float64, device="cuda", requires_grad=True)
+    loss(kappa).backward()
+    ad = float(kappa.grad.cpu().numpy() @ d)
+    eps = 1e-3
+    lp, lm = (float(loss(torch.tensor(kappa0 + s * eps * d, device="cuda"))) for s in (1, -1))
+    fd = (lp - lm) / (2 * eps)
+    _say("  adjoint %.9e fd %.9e" % (ad, fd))
+    assert abs(ad - fd) <= 1e-4 * abs(fd)
