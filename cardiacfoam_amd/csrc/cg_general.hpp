@@ -58,6 +58,14 @@ hipError_t general_rhs0(GeneralMesh* G, const double* Vn, const double* Vm1,
 // face fluxes); asynchronous on s
 hipError_t general_rhs_corr(GeneralMesh* G, const double* psi, const double* b0, double* b,
                             hipStream_t s);
+// the same with the right-hand side in one pass, for a step of a single solve: b = rhs0 + the
+// correction of Vn (whose gradient general_gradient made before), psi = the guess below and
+// its sums per block into xs [blocks] (blocks of RBS threads).  Asynchronous on s
+hipError_t general_rhs(GeneralMesh* G, const double* Vn, const double* Vm1, const double* Iion,
+                       double* psi, double* b, bool extrapolate, double* xs, unsigned blocks,
+                       const GeneralStep& st, hipStream_t s);
+// grad V into the mesh's own buffer; asynchronous on s
+hipError_t general_gradient(GeneralMesh* G, const double* V, hipStream_t s);
 // initial guess of the solve: Vn, or 2 Vn - Vm1 (extrapolate); asynchronous on s
 hipError_t general_guess(GeneralMesh* G, const double* Vn, const double* Vm1, double* psi,
                          bool extrapolate, hipStream_t s);

@@ -30,6 +30,7 @@
 #include <hip/hip_runtime.h>
 
 #include "cg_general.hpp"
+#include "cg_reduce.hpp"
 
 namespace cg {
 
@@ -206,6 +207,33 @@ __global__ __launch_bounds__(GBS) void k_grhs_corr(GView g, const double* __rest
     const int64_t c = (int64_t)blockIdx.x * GBS + threadIdx.x;
     if (c >= g.n) return;
     b[c] = b0[c] + flux_sum(g, psi, grad, c, psi[c], false);
+}
+
+// right-hand side with the correction, initial guess and the guess's block sums: one pass
+// over Vn, its gradient and the faces for the three kernels above and the mean of the guess
+__global__ __launch_bounds__(RBS) void k_grhs(GView g, const double* __restrict__ Vn,
+                                              const double* __restrict__ Vm1,
+                                              const double* __restrict__ Iion,
+                                              const double* __restrict__ grad,
+                                              double* __restrict__ psi, double* __restrict__ b,
+                                              int extrapolate, double* __restrict__ xs,
+                                              GeneralStep st)
+{
+    double v[1] = {0.0};
+    for (int64_t c = (int64_t)blockIdx.x * RBS + threadIdx.x; c < g.n;
+         c += (int64_t)gridDim.x * RBS) {
+        const double vn = Vn[c];
+        const double vo = st.c00 != 0.0 || extrapolate ? Vm1[c] : 0.0;
+        const double src = st.src ? st.src[c] : general_box(g, c, st.boxes);
+        const double b0 = g.vol[c] * (st.chiCm / st.dt * (st.c0 * vn - st.c00 * vo) -
+                                      st.chiCm * Iion[c] + src);
+        b[c] = b0 + flux_sum(g, Vn, grad, c, vn, false);
+        const double p = extrapolate ? 2.0 * vn - vo : vn;
+        psi[c] = p;
+        v[0] += p;
+    }
+    block_sum<RBS, 1>(v);
+    if (threadIdx.x == 0) xs[blockIdx.x] = v[0];
 }
 
 __global__ __launch_bounds__(GBS) void k_gguess(int64_t n, const double* __restrict__ Vn,
@@ -635,6 +663,21 @@ hipError_t general_rhs_corr(GeneralMesh* G, const double* psi, const double* b0,
     hipLaunchKernelGGL(k_ggrad, dim3(grid_of(G->n)), dim3(GBS), 0, s, g, psi, G->grad);
     hipLaunchKernelGGL(k_grhs_corr, dim3(grid_of(G->n)), dim3(GBS), 0, s, g, psi,
                        (const double*)G->grad, b0, b);
+    return hipGetLastError();
+}
+
+hipError_t general_gradient(GeneralMesh* G, const double* V, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_ggrad, dim3(grid_of(G->n)), dim3(GBS), 0, s, G->view(), V, G->grad);
+    return hipGetLastError();
+}
+
+hipError_t general_rhs(GeneralMesh* G, const double* Vn, const double* Vm1, const double* Iion,
+                       double* psi, double* b, bool extrapolate, double* xs, unsigned blocks,
+                       const GeneralStep& st, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_grhs, dim3(blocks), dim3(RBS), 0, s, G->view(), Vn, Vm1, Iion,
+                       (const double*)G->grad, psi, b, extrapolate ? 1 : 0, xs, st);
     return hipGetLastError();
 }
 
