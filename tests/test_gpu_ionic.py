@@ -116,3 +116,22 @@ def test_mixed_state_round_trip(gpu, orc):
     # K_i ~ 145 mM stored as an offset from 145: error ~ulp(offset), not ulp(145) = 1.5e-5
     assert np.max(np.abs(got[4] - states[4])) < 2e-6
     np.testing.assert_allclose(got[1:], states[1:], rtol=2e-7, atol=1e-12)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("n", [1, 524287, 524289])
+def test_states_round_trip_in_pieces(gpu, orc, precision, n):
+    """get_states copies in pieces of 524288 values on several threads: every value of every
+    state comes back, whole arrays and a range of states, one cell to one past a piece.
+    Mixed: half an FP32 ulp (6e-8) of a value, or of its offset from its reference."""
+    _say("states in pieces", precision, n)
+    ion = gpu.IonicModel("TNNP", "epicardialCells", n, precision=precision)
+    ref = ion.states()[:, :1]
+    want = ref + np.random.default_rng(n).uniform(-1e-3, 1e-3, (ion.nstates, n))
+    ion.set_states(want)
+    got, part = ion.states(), ion.states(3, 5)
+    np.testing.assert_array_equal(got[3:8], part)
+    if precision == "fp64":
+        np.testing.assert_array_equal(got, want)
+    else:
+        assert np.all(np.abs(got - want) <= 6e-8 * np.abs(want) + 1e-12)
