@@ -294,7 +294,7 @@ template <class T, bool ADAPTIVE> struct BatchLaunch {
     {
         const unsigned grid = (unsigned)((a.n + BLOCK - 1) / BLOCK);
         hipLaunchKernelGGL((k_cells_protocol<M, T, BLOCK, WPE, INTEG>), dim3(grid), dim3(BLOCK),
-                           0, s, (T*)states, kparams<T>(P), (const T*)gscale, tissue, a);
+                           0, s, (T*)states, kparams<M, T>(P, a.dt), (const T*)gscale, tissue, a);
         return hipGetLastError();
     }
     // the adaptive integrators run one shape, one wave per block (the lanes of a wave take

@@ -1687,6 +1687,7 @@ int cg_tissue_step(cg_tissue* t, int n_steps)
         if (ode0.method) model_step_times(ion->model, t0, dt, &st.ode.t0, &st.ode.t1);
         return st;
     };
+    // Iion is read between calls only: the steps before the last do not store it
     bool ionic_queued = false;  // this step's ionic launch was queued by the previous one
     for (int s = 0; s < n_steps; ++s) {
         const double tn = t->t + dt;
@@ -1698,16 +1699,19 @@ int cg_tissue_step(cg_tissue* t, int n_steps)
         if (t->cfg.algorithm == CG_EXPLICIT) {
             const int tk = prof ? prof->begin(cg::K_IONIC) : -1;
             HIPCHK(cg::launch_explicit_hex(ion->model, ion->prec, ion->tissue, m->g, coefs,
-                                           ion->d_states, Vn, Vm1, Vnew, t->d_Iion, t->d_flag,
+                                           ion->d_states, Vn, Vm1, Vnew,
+                                           s + 1 < n_steps ? nullptr : t->d_Iion, t->d_flag,
                                            t->d_tact, st, ion->P, ion->stream));
             if (prof) prof->end(tk);
         } else {
             cg::NextIonic nx;
             const bool more = s + 1 < n_steps;
             if (more) nx.st = make_step(tn, t->steps + 1);
+            if (s + 2 >= n_steps) nx.Iion = t->d_Iion;
             int rc = cg::implicit_step(t->implicit, ion->model, ion->prec, ion->tissue,
-                                       ion->d_states, ion->P, Vn, Vm1, Vnew, t->d_Iion,
-                                       t->d_flag, t->d_tact, st, t->cfg.tol, t->cfg.max_iter,
+                                       ion->d_states, ion->P, Vn, Vm1, Vnew,
+                                       more ? nullptr : t->d_Iion, t->d_flag, t->d_tact, st,
+                                       t->cfg.tol, t->cfg.max_iter,
                                        prof, ionic_queued, more ? &nx : nullptr,
                                        t->steps >= 1, &g_err);
             if (rc != 0) return rc;

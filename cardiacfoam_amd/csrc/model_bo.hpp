@@ -6,6 +6,13 @@
 // Every gate of this model relaxes as (xinf - x)/tau with (xinf, tau) that depend on u
 // only, so with u held at V^n for the step the Rush-Larsen update is the exact solution
 // of the reference's gate ODEs.
+//
+// What bounds a step: the latency of its chain on a small mesh, instruction issue on a large
+// one.  Gate factors with a constant tau come from the launch (step_factors), an adaptive
+// solver's stages share what depends on u alone (VTerms), and the fused kernel issues the
+// stencil's loads with the gates'.  Explicit kernel, FP64: 147k cells 7.0 -> 4.5 us, 3k cells
+// 4.6 -> 3.8 us, RKF45 on 52k cells 8.2 -> 6.2 us (least of a run, with the division of
+// cg_f64.hpp).
 #pragma once
 #include "cg_common.hpp"
 
@@ -17,7 +24,9 @@ struct BuenoOrovio {
     static constexpr double VSCALE = 85.7, VOFF = 84.0, ISCALE = 85.7, VMUL = 1000.0;
     static constexpr double TSCALE = 1000.0;  // model ms per second
     enum { uo, uu, thv, thw, thvm, tho, tv1m, tv2m, tvp, tw1m, tw2m, kwm, uwm, twp, tfi,
-           to1, to2, tso1, tso2, kso, uso, ts1, ts2, ks, us, tsi, twinf, winfstar };
+           to1, to2, tso1, tso2, kso, uso, ts1, ts2, ks, us, tsi, twinf, winfstar,
+           // a launch's step factors (step_factors), beside the constants
+           Evp, Ev1m, Ev2m, Ewp, Es1, Es2 };
 
     static bool host_init(int tissue, double* p, double* y)
     {
@@ -49,40 +58,79 @@ struct BuenoOrovio {
         return jfi + jso + jsi;
     }
 
-    // Rates of v, w, s at u = y[0] (BuenoOrovio_2008.H:189-220), through an update policy.
-    template <class T, class U> CG_HD static void gate_rates(const T* y, U& out, const T* p)
+    // What the rates of v, w, s at u take from u alone (BuenoOrovio_2008.H:189-220): the
+    // targets and 1/tau.  An adaptive solver of a tissue step, whose u is held, forms them
+    // once for all its stages.
+    template <class T> struct VTerms {
+        T vinf, winf, sinf, rtv, rtw, rts;
+    };
+    template <class T> CG_HD static VTerms<T> vterms(T u, const T* p)
     {
-        const T u = y[0];
         const bool Hv = pos(u - p[thv]), Hw = pos(u - p[thw]), Ho = pos(u - p[tho]),
                    Hvm = pos(u - p[thvm]);
+        VTerms<T> q;
         // v: relaxes to 0 with tau_v+ above theta_v, else to H(theta_v- - u) with tau_v-
-        const T vinf = Hv ? T(0) : (pos(p[thvm] - u) ? T(1) : T(0));
-        const T tv = Hv ? p[tvp] : (Hvm ? p[tv2m] : p[tv1m]);
+        q.vinf = Hv ? T(0) : (pos(p[thvm] - u) ? T(1) : T(0));
+        q.rtv = T(1) / (Hv ? p[tvp] : (Hvm ? p[tv2m] : p[tv1m]));
         // w: relaxes to 0 with tau_w+ above theta_w, else to w_inf with tau_w-
-        const T twm = p[tw1m] + (p[tw2m] - p[tw1m]) * half_1p_tanh(p[kwm] * (u - p[uwm]));
-        const T winf = Hw ? T(0) : (Ho ? p[winfstar] : T(1) - u / p[twinf]);
-        const T tw = Hw ? p[twp] : twm;
+        q.winf = Hw ? T(0) : w_inf(u, Ho, p);
+        q.rtw = T(1) / (Hw ? p[twp] : tau_wm(u, p));
         // s
-        const T sinf = half_1p_tanh(p[ks] * (u - p[us]));
-        const T ts = Hw ? p[ts2] : p[ts1];
-        out.gate(1, vinf, tv);
-        out.gate(2, winf, tw);
-        out.gate(3, sinf, ts);
+        q.sinf = half_1p_tanh(p[ks] * (u - p[us]));
+        q.rts = T(1) / (Hw ? p[ts2] : p[ts1]);
+        return q;
+    }
+    template <class T> CG_HD static T tau_wm(T u, const T* p)
+    {
+        return p[tw1m] + (p[tw2m] - p[tw1m]) * half_1p_tanh(p[kwm] * (u - p[uwm]));
+    }
+    template <class T> CG_HD static T w_inf(T u, bool Ho, const T* p)
+    {
+        return Ho ? p[winfstar] : T(1) - u / p[twinf];
+    }
+
+    // The Rush-Larsen factors of the gates whose tau takes one of a few constants, filled in
+    // for a step of dt beside the constants (Evp..Es2): exp(-dt/tau) for FP64, 1 - exp(-dt/tau)
+    // for FP32 (the form its increments use).  Two of a step's three gate exponentials and
+    // their divisions become selects.
+    template <class T> static void step_factors(double dt, T* p)
+    {
+        const int tau[6] = {tvp, tv1m, tv2m, twp, ts1, ts2};
+        for (int k = 0; k < 6; ++k) {
+            const double e = -dt / double(p[tau[k]]);
+            p[Evp + k] = T(is_fp32<T>() ? -std::expm1(e) : std::exp(e));
+        }
+    }
+    template <class T> CG_HD static T relax(T x, T xinf, T f)
+    {
+        if constexpr (is_fp32<T>()) return x + (xinf - x) * f;
+        else return xinf + (x - xinf) * f;
     }
 
     // Advance v, w, s by dt with u frozen; y[0] is u.
     template <class T> CG_HD static void gates(T* y, T dt, const T* p)
     {
-        RlStep<T> out{y, dt};
-        gate_rates(y, out, p);
+        const T u = y[0];
+        const bool Hv = pos(u - p[thv]), Hw = pos(u - p[thw]), Ho = pos(u - p[tho]),
+                   Hvm = pos(u - p[thvm]);
+        y[1] = relax(y[1], Hv ? T(0) : (pos(p[thvm] - u) ? T(1) : T(0)),
+                     Hv ? p[Evp] : (Hvm ? p[Ev2m] : p[Ev1m]));
+        const T e = dt / tau_wm(u, p);
+        T fw;
+        if constexpr (is_fp32<T>()) fw = rl_frac(e);
+        else fw = cexp(-e);
+        y[2] = relax(y[2], Hw ? T(0) : w_inf(u, Ho, p), Hw ? p[Ewp] : fw);
+        y[3] = relax(y[3], half_1p_tanh(p[ks] * (u - p[us])), Hw ? p[Es2] : p[Es1]);
     }
 
     // dy/dt; du/dt = -Jion - Istim when u is integrated with the gates, else 0
     template <class T>
-    CG_HD static void deriv(const T* y, T* d, const T* p, bool solve_v, T istim)
+    CG_HD static void deriv(const T* y, T* d, const T* p, bool solve_v, T istim,
+                            const VTerms<T>& q)
     {
-        Deriv<T> out{y, d};
-        gate_rates(y, out, p);
+        d[1] = (q.vinf - y[1]) * q.rtv;
+        d[2] = (q.winf - y[2]) * q.rtw;
+        d[3] = (q.sinf - y[3]) * q.rts;
         d[0] = solve_v ? -jion(y[0], y, p) - istim : T(0);
     }
 

@@ -42,6 +42,14 @@ template <class T> inline KParams<T> kparams(const ModelParams& P)
     return k;
 }
 
+// the same for a launch of steps of dt (model time)
+template <class M, class T> inline KParams<T> kparams(const ModelParams& P, double dt)
+{
+    KParams<T> k = kparams<T>(P);
+    if constexpr (std::is_same_v<M, BuenoOrovio>) BuenoOrovio::step_factors<T>(dt, k.p);
+    return k;
+}
+
 // states of one cell: state q of cell c at st[q*n + c], walked with a pointer step of n
 template <int NS, class T>
 CG_DEV void load_states(T (&y)[NS], const T* __restrict__ st, int64_t n, int64_t c, int first)
@@ -319,6 +327,7 @@ CG_DEV double box_source(int i, int j, int k, int64_t c, const HexGeom& g, const
 // monodomainSolver.C:103-118): box stimulus -> ionic step at V^n -> diagonal solve
 //   V^{n+1} = (c0 V^n - c00 V^{n-1} + dt/chiCm (lap - chiCm Iion + src)) / c
 // -> activation time where V first exceeds 1e-15 V (myocardiumDomain.C:345-374).
+// Iion may be null (a step whose Iion nothing reads).
 // Bytes per cell-step (fp64, BuenoOrovio): V 8 + gates 24 r/w + V^{n+1} 8 + Iion 8 +
 // flag 1 (+ V^{n-1} 8 for backward, + off-diagonal sigma 24 with a tensor correction).
 template <class M, class T, bool UNIFORM, int INTEG>
@@ -337,20 +346,24 @@ __global__ __launch_bounds__(MBS) void k_explicit_hex(
     T y[M::NS], sw[M::NS];
     load_model_states<M>(y, sw, st, n, c, 1);
     const double vn = V[c];
+    // the diffusion part before the model's arithmetic, so that one wait covers the state's
+    // and the stencil's loads (a step of a small mesh is the latency of its chain)
+    double lap = hex_laplacian<UNIFORM>(V, c, ix, g, a);
+    if (s.od) lap += hex_tensor_correction(V, s.od, n, c, ix.i, ix.j, ix.k, g, s.od_mask);
+    const double vo = s.c00 != 0.0 ? Vold[c] : 0.0;
+    const uint8_t fl = flag[c];
+    const double src = box_source(ix.i, ix.j, ix.k, c, g, s.boxes);
     const T v = model_v<M, T>(vn);
     const T I = tissue_advance<M, T, INTEG>(v, y, sw, T(s.dt_model), p, tissue, one, s.ode, c);
     store_states(sw, st, n, c, 1);
     const double iion = double(I) * M::ISCALE;
     if (Iion) Iion[c] = iion;
 
-    double lap = hex_laplacian<UNIFORM>(V, c, ix, g, a);
-    if (s.od) lap += hex_tensor_correction(V, s.od, n, c, ix.i, ix.j, ix.k, g, s.od_mask);
-    const double src = box_source(ix.i, ix.j, ix.k, c, g, s.boxes);
-    double rhs = s.c0 * vn + s.dt / s.chiCm * (lap - s.chiCm * iion + src);
-    if (s.c00 != 0.0) rhs -= s.c00 * Vold[c];
-    const double vnew = rhs / s.c;
+    double rhs = s.c0 * vn + div_f64(s.dt, s.chiCm) * (lap - s.chiCm * iion + src);
+    if (s.c00 != 0.0) rhs -= s.c00 * vo;
+    const double vnew = div_f64(rhs, s.c);
     Vnew[c] = vnew;
-    if (flag[c] && vnew > s.act_v + 1e-15) {
+    if (fl && vnew > s.act_v + 1e-15) {
         flag[c] = 0;
         tact[c] = s.t_old + (s.act_v - vn) / (vnew - vn) * s.dt;
     }
@@ -358,7 +371,7 @@ __global__ __launch_bounds__(MBS) void k_explicit_hex(
 
 // ------------------------------------------ ionic step + implicit right-hand side
 // rhs = chiCm/dt (c0 V^n - c00 V^{n-1}) - chiCm Iion + source (the explicit tensor
-// correction is added by the solver's first residual); x0 (when not null) receives the
+// correction is added by the solver's first residual); Iion may be null; x0 (when not null) receives the
 // solver's extrapolated initial guess 2 V^n - V^{n-1}, riding on this kernel's pass over
 // V^n; with s.act_flag it also completes the previous step's activation times.  With a
 // gate (s.gate) the launch may be queued before the previous step's solve is known to have
@@ -401,9 +414,9 @@ void k_ionic_rhs(HexGeom g, T* __restrict__ st,
     const T I = tissue_advance<M, T, INTEG>(v, y, sw, T(s.dt_model), p, tissue, one, s.ode, c);
     store_states(sw, st, n, c, 1);
     const double iion = double(I) * M::ISCALE;
-    Iion[c] = iion;
+    if (Iion) Iion[c] = iion;
     const double src = box_source(cc.i, cc.j, cc.k, c, g, s.boxes);
-    double rhs = s.chiCm / s.dt * (s.c0 * vn - s.c00 * vo) + src - s.chiCm * iion;
+    double rhs = div_f64(s.chiCm, s.dt) * (s.c0 * vn - s.c00 * vo) + src - s.chiCm * iion;
     b[c] = rhs;
     if (x0) x0[c] = 2.0 * vn - vo;
     // the previous step's activation: V^n is its new potential, V^{n-1} its old one
@@ -465,7 +478,7 @@ template <class T, bool ADAPTIVE> struct ModelLaunch {
         const unsigned grid = (unsigned)((n + MBS - 1) / MBS);
 #define CG_IONIC_TISSUE(I)                                                                 \
     hipLaunchKernelGGL((k_ionic_tissue<M, T, I>), dim3(grid), dim3(MBS), 0, s, (T*)states, \
-                       n, Vm, Im, T(dt_model), kparams<T>(P), (const T*)gscale, tissue, ode)
+                       n, Vm, Im, T(dt_model), kparams<M, T>(P, dt_model), (const T*)gscale, tissue, ode)
         if constexpr (!ADAPTIVE) CG_IONIC_TISSUE(0);
         else if (ode.method == 2) CG_IONIC_TISSUE(2);
         else CG_IONIC_TISSUE(1);
@@ -481,7 +494,7 @@ template <class T, bool ADAPTIVE> struct ModelLaunch {
         const unsigned grid = (unsigned)((n + MBS - 1) / MBS);
 #define CG_IONIC_CELLS(I)                                                                  \
     hipLaunchKernelGGL((k_ionic_cells<M, T, I>), dim3(grid), dim3(MBS), 0, s, (T*)states,  \
-                       n, t0, T(dt), n_steps, kparams<T>(P), (const T*)gscale, tissue, stim, \
+                       n, t0, T(dt), n_steps, kparams<M, T>(P, dt), (const T*)gscale, tissue, stim, \
                        ode, trace, tcell)
         if constexpr (!ADAPTIVE) CG_IONIC_CELLS(0);
         else if (ode.method == 2) CG_IONIC_CELLS(2);
@@ -499,7 +512,8 @@ template <class T, bool ADAPTIVE> struct ModelLaunch {
         const unsigned grid = (unsigned)((n + MBS - 1) / MBS);
 #define CG_EXPLICIT_HEX(U, I)                                                              \
     hipLaunchKernelGGL((k_explicit_hex<M, T, U, I>), dim3(grid), dim3(MBS), 0, s, g, a,    \
-                       (T*)states, V, Vold, Vnew, Iion, flag, tact, st, kparams<T>(P), tissue)
+                       (T*)states, V, Vold, Vnew, Iion, flag, tact, st,                    \
+                       kparams<M, T>(P, st.dt_model), tissue)
         if constexpr (!ADAPTIVE) {
             if (a.fx) CG_EXPLICIT_HEX(false, 0);
             else CG_EXPLICIT_HEX(true, 0);
@@ -522,7 +536,8 @@ template <class T, bool ADAPTIVE> struct ModelLaunch {
         const int64_t n = (int64_t)g.nx * g.ny * g.nz;
 #define CG_IONIC_RHS(I)                                                                    \
     hipLaunchKernelGGL((k_ionic_rhs<M, T, I>), dim3(grid_8(n, MBS)), dim3(MBS), 0, s, g,    \
-                       (T*)states, Vn, Vm1, x0, Iion, b, st, kparams<T>(P), tissue)
+                       (T*)states, Vn, Vm1, x0, Iion, b, st, kparams<M, T>(P, st.dt_model), \
+                       tissue)
         if constexpr (!ADAPTIVE) CG_IONIC_RHS(0);
         else if (st.ode.method == 2) CG_IONIC_RHS(2);
         else CG_IONIC_RHS(1);

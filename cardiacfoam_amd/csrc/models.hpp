@@ -161,13 +161,15 @@ template <> struct Ops<BuenoOrovio> {
     {
         return BuenoOrovio::jion(y[0], y, p);
     }
-    struct None {};
-    template <class T> CG_HD static None vt(T, const T*) { return None{}; }
+    template <class T> CG_HD static BuenoOrovio::VTerms<T> vt(T u, const T* p)
+    {
+        return BuenoOrovio::vterms(u, p);
+    }
     template <class T>
     CG_HD static void deriv(const T* y, T* d, const T* p, int, const T*, bool solve_v, T istim,
-                             None)
+                             const BuenoOrovio::VTerms<T>& q)
     {
-        BuenoOrovio::deriv(y, d, p, solve_v, istim);
+        BuenoOrovio::deriv(y, d, p, solve_v, istim, q);
     }
 };
 

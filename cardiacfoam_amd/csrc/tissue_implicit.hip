@@ -1368,8 +1368,8 @@ int implicit_step(ImplicitSolver* S, int model, int prec, int tissue, void* stat
             S->x0_in_new = prec == 0 && S->next_even;
             double* x0 = !fuse || !(prec == 1 || use_cheb(sn.c)) ? nullptr
                          : S->x0_in_new ? const_cast<double*>(Vm1) : S->xalt;
-            launch_ionic_rhs(model, prec, tissue, S->g, states, Vnew, Vn, x0, Iion, S->b, sn,
-                             P, S->stream);
+            launch_ionic_rhs(model, prec, tissue, S->g, states, Vnew, Vn, x0, next->Iion, S->b,
+                             sn, P, S->stream);
             if (prof) prof->end(t);
         }
         if (hipGetLastError() != hipSuccess) return false;
