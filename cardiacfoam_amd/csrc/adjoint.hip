@@ -45,9 +45,12 @@ constexpr int AG = 1024;  // blocks of the backward kernel (parameter partials)
 
 using BO = BuenoOrovio;
 
-// slot layout of the state store: V, v, w, s, then the step's transcendental factors
-// exp(-dt/tau_v), exp(-dt/tau_w), exp(-dt/tau_s), tanh of tau_w-, s_inf and tau_so
-enum { SL_V, SL_v, SL_w, SL_s, SL_Ev, SL_Ew, SL_Es, SL_thw, SL_ths, SL_thso, SL_N };
+// slot layout of the state store.  The backward kernel forms the step's transcendental
+// factors again from V (four exponentials): storing them took 48 of the forward kernel's
+// 136 B per cell and the same of the backward's, and made the store of a 150-step run of
+// 131k cells 1.6 GB, six times the last-level cache.  131k cells: forward kernel 9.1 ->
+// 6.1 us, backward 8.6 -> 7.7 us.
+enum { SL_V, SL_v, SL_w, SL_s, SL_N };
 
 // stimulus boxes of the tissue (myocardiumDomain.C:307-342), active when the step start
 // t0 lies in [t_start, t_start + duration]
@@ -63,7 +66,7 @@ struct AdjGeom {
     const double* fx;   // face coefficients a_f (per unit volume), + faces, 0 on walls
     const double* fy;
     const double* fz;
-    const double* prm;  // BuenoOrovio constants (device)
+    const F64* prm;     // BuenoOrovio constants and step factors (device)
     const BoxTable* boxes;
     double dt, dt_model, chiCm;
 };
@@ -85,44 +88,47 @@ CG_DEV double box_src(int i, int j, int k, const HexGeom& g, const BoxTable& b, 
     return src;
 }
 
-// The BuenoOrovio tissue step (u frozen) written out with its transcendental factors,
-// operation for operation as BuenoOrovio::gates and ::jion; returns Jion at the step end.
+// What a step at u takes its gates and currents from: the Rush-Larsen factors, and the
+// sigmoids (1 + tanh x)/2 of tau_w-, s_inf and tau_so.
 struct BoFactors {
-    double Ev, Ew, Es, thw, ths, thso;
+    F64 Ev, Ew, Es, sgw, sgs, sgso;
 };
-CG_DEV double bo_step(double u, double& v, double& w, double& s, double dt, const double* p,
-                      BoFactors& f)
+CG_DEV BoFactors bo_factors(F64 u, F64 dt, const F64* p)
 {
-    const bool Hv = pos(u - p[BO::thv]), Hw = pos(u - p[BO::thw]), Ho = pos(u - p[BO::tho]),
-               Hvm = pos(u - p[BO::thvm]);
-    const double vinf = Hv ? 0.0 : (pos(p[BO::thvm] - u) ? 1.0 : 0.0);
-    const double tv = Hv ? p[BO::tvp] : (Hvm ? p[BO::tv2m] : p[BO::tv1m]);
-    f.thw = tanh(p[BO::kwm] * (u - p[BO::uwm]));
-    const double twm = p[BO::tw1m] + (p[BO::tw2m] - p[BO::tw1m]) * (1.0 + f.thw) / 2.0;
-    const double winf = Hw ? 0.0 : (Ho ? p[BO::winfstar] : 1.0 - u / p[BO::twinf]);
-    const double tw = Hw ? p[BO::twp] : twm;
-    f.ths = tanh(p[BO::ks] * (u - p[BO::us]));
-    const double sinf = (1.0 + f.ths) / 2.0;
-    const double ts = Hw ? p[BO::ts2] : p[BO::ts1];
-    f.Ev = exp(-dt / tv);
-    f.Ew = exp(-dt / tw);
-    f.Es = exp(-dt / ts);
-    v = vinf + (v - vinf) * f.Ev;
-    w = winf + (w - winf) * f.Ew;
-    s = sinf + (s - sinf) * f.Es;
-    f.thso = tanh(p[BO::kso] * (u - p[BO::uso]));
-    const double tso = p[BO::tso1] + (p[BO::tso2] - p[BO::tso1]) * (1.0 + f.thso) / 2.0;
-    const double to = Ho ? p[BO::to2] : p[BO::to1];
-    const double jfi = Hv ? -v * (u - p[BO::thv]) * (p[BO::uu] - u) / p[BO::tfi] : 0.0;
-    const double jso = Hw ? 1.0 / tso : (u - p[BO::uo]) / to;
-    const double jsi = Hw ? -w * s / p[BO::tsi] : 0.0;
-    return jfi + jso + jsi;
+    const bool Hv = pos(u - p[BO::thv]), Hw = pos(u - p[BO::thw]), Hvm = pos(u - p[BO::thvm]);
+    BoFactors f;
+    f.sgw = half_1p_tanh(p[BO::kwm] * (u - p[BO::uwm]));
+    f.sgs = half_1p_tanh(p[BO::ks] * (u - p[BO::us]));
+    f.sgso = half_1p_tanh(p[BO::kso] * (u - p[BO::uso]));
+    f.Ev = Hv ? p[BO::Evp] : (Hvm ? p[BO::Ev2m] : p[BO::Ev1m]);
+    f.Es = Hw ? p[BO::Es2] : p[BO::Es1];
+    const F64 ew = cexp(-(dt / (p[BO::tw1m] + (p[BO::tw2m] - p[BO::tw1m]) * f.sgw)));
+    f.Ew = Hw ? p[BO::Ewp] : ew;
+    return f;
 }
 
+// The BuenoOrovio tissue step (u frozen) with its factors, operation for operation as
+// BuenoOrovio::gates and ::jion; returns Jion at the step end.
+CG_DEV F64 bo_step(F64 u, F64& v, F64& w, F64& s, const F64* p, const BoFactors& f)
+{
+    const bool Hv = pos(u - p[BO::thv]), Hw = pos(u - p[BO::thw]), Ho = pos(u - p[BO::tho]);
+    const F64 vinf = Hv ? F64(0.0) : (pos(p[BO::thvm] - u) ? F64(1.0) : F64(0.0));
+    const F64 winf = Hw ? F64(0.0) : BO::w_inf(u, Ho, p);
+    v = BO::relax(v, vinf, f.Ev);
+    w = BO::relax(w, winf, f.Ew);
+    s = BO::relax(s, f.sgs, f.Es);
+    const F64 tso = p[BO::tso1] + (p[BO::tso2] - p[BO::tso1]) * f.sgso;
+    const F64 to = Ho ? p[BO::to2] : p[BO::to1];
+    const F64 jfi = Hv ? -v * (u - p[BO::thv]) * (p[BO::uu] - u) / p[BO::tfi] : F64(0.0);
+    const F64 jso = Hw ? F64(1.0) / tso : (u - p[BO::uo]) / to;
+    const F64 jsi = Hw ? -w * s / p[BO::tsi] : F64(0.0);
+    return jfi + jso + jsi;
+}
+CG_DEV F64 bo_u(double v) { return F64(v * 1000.0 + BO::VOFF) / F64(BO::VSCALE); }
+
 // ------------------------------------------------------------------ forward
-// One step from slot `in` into slot `out` (planes SL_V..SL_s, [plane][n]); when aux is
-// not null (planes SL_Ev.. of the input slot) the step's factors are stored there; Vm at
-// probes into probe_row.
+// One step from slot `in` into slot `out` (planes SL_V..SL_s, [plane][n]); Vm at probes into
+// probe_row.
 // IMPL: the diffusion is implicit; instead of V^{n+1} the kernel writes the right-hand
 // side V - dt I + a src of M V^{n+1} into bvec and V^n (the solve's initial guess) into the
 // output V plane, and records no probes (the solve's result is V^{n+1}).
@@ -130,7 +136,6 @@ template <bool IMPL>
 __global__ __launch_bounds__(ABS) void k_adj_forward(AdjGeom G, double t0,
                                                      const double* __restrict__ in,
                                                      double* __restrict__ out,
-                                                     double* __restrict__ aux,
                                                      const int* __restrict__ probe_slot,
                                                      double* __restrict__ probe_row,
                                                      double* __restrict__ bvec)
@@ -140,31 +145,25 @@ __global__ __launch_bounds__(ABS) void k_adj_forward(AdjGeom G, double t0,
     const int64_t c = (int64_t)blockIdx.x * ABS + threadIdx.x;
     if (c >= n) return;
     const IJK q = ijk_of((uint32_t)c, g);
-    double v = in[SL_v * n + c], w = in[SL_w * n + c], s = in[SL_s * n + c];
+    F64 v = in[SL_v * n + c], w = in[SL_w * n + c], s = in[SL_s * n + c];
     const double vn = in[SL_V * n + c];
-    const double u = (vn * 1000.0 + BO::VOFF) / BO::VSCALE;
-    BoFactors f;
-    const double iion = bo_step(u, v, w, s, G.dt_model, G.prm, f) * BO::ISCALE;
-    out[SL_v * n + c] = v;
-    out[SL_w * n + c] = w;
-    out[SL_s * n + c] = s;
-    if (aux) {  // planes SL_Ev.. of the input slot
-        aux[(SL_Ev - SL_Ev) * n + c] = f.Ev;
-        aux[(SL_Ew - SL_Ev) * n + c] = f.Ew;
-        aux[(SL_Es - SL_Ev) * n + c] = f.Es;
-        aux[(SL_thw - SL_Ev) * n + c] = f.thw;
-        aux[(SL_ths - SL_Ev) * n + c] = f.ths;
-        aux[(SL_thso - SL_Ev) * n + c] = f.thso;
-    }
+    // the stencil's loads beside the gates'
+    const HexCoefs hc{0, 0, 0, G.fx, G.fy, G.fz};
+    const double lap = IMPL ? 0.0 : hex_laplacian<false>(in + SL_V * n, c, q, g, hc);
     const double src = box_src(q.i, q.j, q.k, g, *G.boxes, t0);
+    const F64 u = bo_u(vn);
+    const double iion = double(bo_step(u, v, w, s, G.prm, bo_factors(u, G.dt_model, G.prm))) *
+                        BO::ISCALE;
+    out[SL_v * n + c] = double(v);
+    out[SL_w * n + c] = double(w);
+    out[SL_s * n + c] = double(s);
+    const double a = div_f64(G.dt, G.chiCm);
     if constexpr (IMPL) {
-        bvec[c] = vn + G.dt / G.chiCm * (src - G.chiCm * iion);
+        bvec[c] = vn + a * (src - G.chiCm * iion);
         out[SL_V * n + c] = vn;
         return;
     }
-    const HexCoefs hc{0, 0, 0, G.fx, G.fy, G.fz};
-    const double lap = hex_laplacian<false>(in + SL_V * n, c, q, g, hc);
-    const double vnew = (1.0 * vn + G.dt / G.chiCm * (lap - G.chiCm * iion + src)) / 1.0;
+    const double vnew = vn + a * (lap - G.chiCm * iion + src);
     out[SL_V * n + c] = vnew;
     if (probe_row) {
         const int slot = probe_slot[c];
@@ -192,47 +191,48 @@ __global__ __launch_bounds__(ABS) void k_adj_faces(HexGeom g, const double* __re
 
 // ----------------------------------------------------------------- cell VJP
 struct CellAdj {
-    double lv, lw, ls, lu, dtfi, dtsi;
+    F64 lv, lw, ls, lu, dtfi, dtsi;
 };
 
-// Vector-Jacobian product of bo_step at (u, v, w, s) with its stored factors f: cotangents
-// (lv1, lw1, ls1) of the updated gates and lJ of Jion.  Derivatives by hand from the
-// model equations; the Heaviside switches are piecewise constant (zero derivative).
-CG_DEV CellAdj bo_vjp(double u, double v, double w, double s, const BoFactors& f, double dt,
-                      const double* p, double lv1, double lw1, double ls1, double lJ)
+// Vector-Jacobian product of bo_step at (u, v, w, s) with its factors f: cotangents
+// (lv1, lw1, ls1) of the updated gates and lJ of Jion.  Derivatives by hand from the model
+// equations, d/dx (1 + tanh x)/2 = 2 g (1 - g); the Heaviside switches are piecewise
+// constant (zero derivative).
+CG_DEV CellAdj bo_vjp(F64 u, F64 v, F64 w, F64 s, const BoFactors& f, F64 dt, const F64* p,
+                      F64 lv1, F64 lw1, F64 ls1, F64 lJ)
 {
+    const F64 zero = 0.0, one = 1.0, two = 2.0;
     const bool Hv = pos(u - p[BO::thv]), Hw = pos(u - p[BO::thw]), Ho = pos(u - p[BO::tho]);
-    const double vinf = Hv ? 0.0 : (pos(p[BO::thvm] - u) ? 1.0 : 0.0);
-    const double twm = p[BO::tw1m] + (p[BO::tw2m] - p[BO::tw1m]) * (1.0 + f.thw) / 2.0;
-    const double dtwm = (p[BO::tw2m] - p[BO::tw1m]) * p[BO::kwm] * (1.0 - f.thw * f.thw) / 2.0;
-    const double winf = Hw ? 0.0 : (Ho ? p[BO::winfstar] : 1.0 - u / p[BO::twinf]);
-    const double dwinf = (!Hw && !Ho) ? -1.0 / p[BO::twinf] : 0.0;
-    const double tw = Hw ? p[BO::twp] : twm;
-    const double dtw = Hw ? 0.0 : dtwm;
-    const double sinf = (1.0 + f.ths) / 2.0;
-    const double dsinf = p[BO::ks] * (1.0 - f.ths * f.ths) / 2.0;
-    const double v1 = vinf + (v - vinf) * f.Ev;
-    const double w1 = winf + (w - winf) * f.Ew;
-    const double s1 = sinf + (s - sinf) * f.Es;
-    const double dw1du = dwinf * (1.0 - f.Ew) + (w - winf) * f.Ew * dt / (tw * tw) * dtw;
-    const double ds1du = dsinf * (1.0 - f.Es);
-    const double tfi = p[BO::tfi], tsi = p[BO::tsi];
-    const double a1 = u - p[BO::thv], a2 = p[BO::uu] - u;
-    const double tso = p[BO::tso1] + (p[BO::tso2] - p[BO::tso1]) * (1.0 + f.thso) / 2.0;
-    const double dtso = (p[BO::tso2] - p[BO::tso1]) * p[BO::kso] * (1.0 - f.thso * f.thso) / 2.0;
-    const double to = Ho ? p[BO::to2] : p[BO::to1];
-    const double dJ_dv1 = Hv ? -a1 * a2 / tfi : 0.0;
-    const double dJ_dw1 = Hw ? -s1 / tsi : 0.0;
-    const double dJ_ds1 = Hw ? -w1 / tsi : 0.0;
-    const double dJ_du = (Hv ? -v1 * (a2 - a1) / tfi : 0.0) + (Hw ? -dtso / (tso * tso) : 1.0 / to);
-    const double cv = lv1 + lJ * dJ_dv1, cw = lw1 + lJ * dJ_dw1, cs = ls1 + lJ * dJ_ds1;
+    const F64 vinf = Hv ? zero : (pos(p[BO::thvm] - u) ? one : zero);
+    const F64 twm = p[BO::tw1m] + (p[BO::tw2m] - p[BO::tw1m]) * f.sgw;
+    const F64 dtwm = (p[BO::tw2m] - p[BO::tw1m]) * p[BO::kwm] * (two * f.sgw * (one - f.sgw));
+    const F64 winf = Hw ? zero : BO::w_inf(u, Ho, p);
+    const F64 dwinf = (!Hw && !Ho) ? -one / p[BO::twinf] : zero;
+    const F64 tw = Hw ? p[BO::twp] : twm;
+    const F64 dtw = Hw ? zero : dtwm;
+    const F64 dsinf = p[BO::ks] * (two * f.sgs * (one - f.sgs));
+    const F64 v1 = BO::relax(v, vinf, f.Ev);
+    const F64 w1 = BO::relax(w, winf, f.Ew);
+    const F64 s1 = BO::relax(s, f.sgs, f.Es);
+    const F64 dw1du = dwinf * (one - f.Ew) + (w - winf) * f.Ew * dt / (tw * tw) * dtw;
+    const F64 ds1du = dsinf * (one - f.Es);
+    const F64 rtfi = one / p[BO::tfi], rtsi = one / p[BO::tsi];
+    const F64 a1 = u - p[BO::thv], a2 = p[BO::uu] - u;
+    const F64 tso = p[BO::tso1] + (p[BO::tso2] - p[BO::tso1]) * f.sgso;
+    const F64 dtso = (p[BO::tso2] - p[BO::tso1]) * p[BO::kso] * (two * f.sgso * (one - f.sgso));
+    const F64 to = Ho ? p[BO::to2] : p[BO::to1];
+    const F64 dJ_dv1 = Hv ? -a1 * a2 * rtfi : zero;
+    const F64 dJ_dw1 = Hw ? -s1 * rtsi : zero;
+    const F64 dJ_ds1 = Hw ? -w1 * rtsi : zero;
+    const F64 dJ_du = (Hv ? -v1 * (a2 - a1) * rtfi : zero) + (Hw ? -dtso / (tso * tso) : one / to);
+    const F64 cv = lv1 + lJ * dJ_dv1, cw = lw1 + lJ * dJ_dw1, cs = ls1 + lJ * dJ_ds1;
     CellAdj r;
     r.lv = cv * f.Ev;
     r.lw = cw * f.Ew;
     r.ls = cs * f.Es;
     r.lu = lJ * dJ_du + cw * dw1du + cs * ds1du;  // v1 does not depend on u (a.e.)
-    r.dtfi = Hv ? lJ * v1 * a1 * a2 / (tfi * tfi) : 0.0;
-    r.dtsi = Hw ? lJ * w1 * s1 / (tsi * tsi) : 0.0;
+    r.dtfi = Hv ? lJ * v1 * a1 * a2 * rtfi * rtfi : zero;
+    r.dtsi = Hw ? lJ * w1 * s1 * rtsi * rtsi : zero;
     return r;
 }
 
@@ -257,7 +257,7 @@ template <int NV> CG_DEV void block_sum_a(double (&v)[NV])
 }
 
 // ----------------------------------------------------------------- backward
-// Adjoint of step n from its slot (state and factors of step n).  mu = dLoss/dV^{n+1}
+// Adjoint of step n from its slot (the state of step n).  mu = dLoss/dV^{n+1}
 // (with the probe seed of V^{n+1}), ly1 = dLoss/dy^{n+1}; writes lV = dLoss/dV^n (plus the
 // seed of V^n from seed_row when not null) and ly = dLoss/dy^n, adds into gk and into the
 // per-block parameter partials.  Grid-stride over cells with AG blocks (block b always
@@ -279,7 +279,7 @@ __global__ __launch_bounds__(ABS) void k_adj_backward(AdjGeom G, double gxh, dou
 {
     const HexGeom& g = G.g;
     const int64_t n = (int64_t)g.nx * g.ny * g.nz;
-    const double* __restrict__ p = G.prm;
+    const F64* __restrict__ p = G.prm;
     const double a = G.dt / G.chiCm;
     const double lJ_per_mu = -G.dt * BO::ISCALE;
     const double du_dV = 1000.0 / BO::VSCALE;
@@ -290,26 +290,19 @@ __global__ __launch_bounds__(ABS) void k_adj_backward(AdjGeom G, double gxh, dou
         const Nbr b = nbr_of(c, q, g);
         const double muc = mu[c];
         const double vc = Vn[c];
-        const double u = (vc * 1000.0 + BO::VOFF) / BO::VSCALE;
-        BoFactors f;
-        f.Ev = sl[SL_Ev * n + c];
-        f.Ew = sl[SL_Ew * n + c];
-        f.Es = sl[SL_Es * n + c];
-        f.thw = sl[SL_thw * n + c];
-        f.ths = sl[SL_ths * n + c];
-        f.thso = sl[SL_thso * n + c];
-        const CellAdj r = bo_vjp(u, sl[SL_v * n + c], sl[SL_w * n + c], sl[SL_s * n + c], f,
-                                 G.dt_model, p, ly1[c], ly1[n + c], ly1[2 * n + c],
-                                 lJ_per_mu * muc);
-        ly[c] = r.lv;
-        ly[n + c] = r.lw;
-        ly[2 * n + c] = r.ls;
-        acc[0] += r.dtfi;
-        acc[1] += r.dtsi;
+        const F64 u = bo_u(vc);
+        const CellAdj r = bo_vjp(u, sl[SL_v * n + c], sl[SL_w * n + c], sl[SL_s * n + c],
+                                 bo_factors(u, G.dt_model, p), G.dt_model, p, ly1[c],
+                                 ly1[n + c], ly1[2 * n + c], lJ_per_mu * muc);
+        ly[c] = double(r.lv);
+        ly[n + c] = double(r.lw);
+        ly[2 * n + c] = double(r.ls);
+        acc[0] += double(r.dtfi);
+        acc[1] += double(r.dtsi);
         // diffusion adjoint (L symmetric) and the kappa gradient, one pass over the faces
         const double mxp = mu[b.xp], mxm = mu[b.xm], myp = mu[b.yp], mym = mu[b.ym];
         const double mzp = mu[b.zp], mzm = mu[b.zm];
-        double lv = muc + du_dV * r.lu;
+        double lv = muc + du_dV * double(r.lu);
         if constexpr (!IMPL) {
             const double fxp = G.fx[c], fxm = G.fx[b.xm], fyp = G.fy[c], fym = G.fy[b.ym];
             const double fzp = G.fz[c], fzm = G.fz[b.zm];
@@ -581,7 +574,8 @@ struct Adjoint {
     ModelParams P;
     int K;                      // checkpoint interval
     int n_probes;
-    double* d_prm = nullptr;    // model constants [NP]
+    double* d_prm = nullptr;    // model constants and step factors [MAX_PARAMS]
+    double h_prm[MAX_PARAMS];   // their host copy (source of an asynchronous upload)
     BoxTable* d_boxes = nullptr;
     uint8_t* d_mask = nullptr;  // copy of the tissue's box-membership mask, or null
     int* d_slot = nullptr;      // [n] probe slot or -1
@@ -702,7 +696,7 @@ static AdjGeom geom_of(const Adjoint* A)
     G.fx = A->fx;
     G.fy = A->fy;
     G.fz = A->fz;
-    G.prm = A->d_prm;
+    G.prm = (const F64*)A->d_prm;
     G.boxes = A->d_boxes;
     G.dt = A->dt;
     G.dt_model = A->dt_model;
@@ -808,19 +802,18 @@ static int adj_solve(Adjoint* A, const AdjGeom& G, const double* b, double* x,
     return 0;
 }
 
-// one forward step from slot `in` into slot `outp` (factors into aux, probes into
-// probe_row when not null)
+// one forward step from slot `in` into slot `outp` (probes into probe_row when not null)
 static int adj_step(Adjoint* A, const AdjGeom& G, double t0, const double* in, double* outp,
-                    double* aux, double* probe_row, std::string* err)
+                    double* probe_row, std::string* err)
 {
     const unsigned nb = blocks_of(A->n);
     if (!A->implicit) {
         hipLaunchKernelGGL(k_adj_forward<false>, dim3(nb), dim3(ABS), 0, A->stream, G, t0, in,
-                           outp, aux, (const int*)A->d_slot, probe_row, (double*)nullptr);
+                           outp, (const int*)A->d_slot, probe_row, (double*)nullptr);
         return 0;
     }
     hipLaunchKernelGGL(k_adj_forward<true>, dim3(nb), dim3(ABS), 0, A->stream, G, t0, in,
-                       outp, aux, (const int*)A->d_slot, (double*)nullptr, A->bvec);
+                       outp, (const int*)A->d_slot, (double*)nullptr, A->bvec);
     if (adj_cheb(A))
         adj_solve_cheb(A, G, A->bvec, in + SL_V * A->n, outp + SL_V * A->n);
     else if (int rc = adj_solve(A, G, A->bvec, outp + SL_V * A->n, err))
@@ -877,7 +870,9 @@ int adjoint_forward(Adjoint* A, const double* kappa, const double* theta, const 
         *err = "checkpoint allocation failed";
         return 5;
     }
-    hipMemcpyAsync(A->d_prm, A->P.p, sizeof(double) * MAX_PARAMS, hipMemcpyHostToDevice,
+    for (int i = 0; i < MAX_PARAMS; ++i) A->h_prm[i] = A->P.p[i];
+    BO::step_factors<double>(A->dt_model, A->h_prm);
+    hipMemcpyAsync(A->d_prm, A->h_prm, sizeof(double) * MAX_PARAMS, hipMemcpyHostToDevice,
                    A->stream);
     hipLaunchKernelGGL(k_adj_faces, dim3(nb), dim3(ABS), 0, A->stream, A->g, kappa, A->gx,
                        A->gy, A->gz, A->fx, A->fy, A->fz);
@@ -903,11 +898,9 @@ int adjoint_forward(Adjoint* A, const double* kappa, const double* theta, const 
     for (int st = 0; st < n_steps; ++st) {
         double* in;
         double* outp;
-        double* aux = nullptr;
         if (A->store_all) {
             in = A->seg + (size_t)st * SL_N * n;
             outp = in + (size_t)SL_N * n;
-            aux = in + SL_Ev * n;
         } else {  // two slots in turn, a checkpoint every K steps
             in = A->seg + (size_t)(st & 1) * SL_N * n;
             outp = A->seg + (size_t)((st + 1) & 1) * SL_N * n;
@@ -915,8 +908,7 @@ int adjoint_forward(Adjoint* A, const double* kappa, const double* theta, const 
                 hipMemcpyAsync(A->ck + (size_t)(st / A->K) * 4 * n, in, 8 * 4 * n,
                                hipMemcpyDeviceToDevice, A->stream);
         }
-        if (int rc = adj_step(A, G, t0[st], in, outp, aux, probes + (size_t)st * A->n_probes,
-                              err))
+        if (int rc = adj_step(A, G, t0[st], in, outp, probes + (size_t)st * A->n_probes, err))
             return rc;
     }
     bool missed;
@@ -969,13 +961,12 @@ int adjoint_backward(Adjoint* A, const double* dprobes, double* dkappa, double* 
         const int s0 = sgi * K, s1 = s0 + K < N ? s0 + K : N;
         const double* base = A->store_all ? A->seg + (size_t)s0 * SN : A->seg;
         if (!A->store_all) {
-            // recompute the segment: slot j <- state at step s0 + j, with the factors
+            // recompute the segment: slot j <- state at step s0 + j
             hipMemcpyAsync(A->seg, A->ck + (size_t)sgi * 4 * n, 8 * 4 * n,
                            hipMemcpyDeviceToDevice, A->stream);
             for (int st = s0; st < s1; ++st) {
                 double* in = A->seg + (size_t)(st - s0) * SN;
-                if (int rc = adj_step(A, G, A->t0[st], in, in + SN, in + SL_Ev * n, nullptr,
-                                      err))
+                if (int rc = adj_step(A, G, A->t0[st], in, in + SN, nullptr, err))
                     return rc;
             }
         }
