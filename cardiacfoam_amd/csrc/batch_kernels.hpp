@@ -90,6 +90,7 @@ template <class T> struct Detector {
     double v1, v2, v3, dvp;
     Beat cur, old;
     int nb;
+    int rp;   // ring position of the next sample, s0 % ring_len at the launch's first
 
     CG_DEV double t_of(int64_t j) const { return (double)(j + 1) * a.dt; }
 
@@ -103,6 +104,7 @@ template <class T> struct Detector {
         beat_load(cur, a.det, n, lane, DS_CUR);
         beat_load(old, a.det, n, lane, DS_OLD);
         nb = a.nbeats[cell];
+        rp = (int)(a.s0 % a.ring_len);
     }
     CG_DEV void store()
     {
@@ -116,17 +118,21 @@ template <class T> struct Detector {
         a.nbeats[cell] = nb;
     }
 
-    // min of the ring samples with t in [tu - baseline, tu); samples up to index i held
+    // min of the ring samples with t in [tu - baseline, tu); samples up to index i held, i at
+    // position rp
     CG_DEV bool baseline(int64_t i, double tu, double& vmin) const
     {
         bool any = false;
         vmin = __builtin_inf();
         const int64_t lo = i - a.ring_len + 1 > 0 ? i - a.ring_len + 1 : 0;
+        int r = rp;
         for (int64_t j = i; j >= lo; --j) {
+            const int at = r;
+            r = r == 0 ? a.ring_len - 1 : r - 1;
             const double tj = t_of(j);
             if (tj >= tu) continue;
             if (tj < tu - a.baseline) break;
-            const double v = (double)ring[(j % a.ring_len) * a.n + lane];
+            const double v = (double)ring[at * a.n + lane];
             if (v < vmin) vmin = v;
             any = true;
         }
@@ -145,9 +151,9 @@ template <class T> struct Detector {
     // sample i (value vi) after step i + 1
     CG_DEV void push(int64_t i, double vi)
     {
-        ring[(i % a.ring_len) * a.n + lane] = T(vi);
+        ring[rp * a.n + lane] = T(vi);
         if (i >= 2) {
-            const double dv = (vi - v2) / (t_of(i) - t_of(i - 2));
+            const double dv = div_f64(vi - v2, t_of(i) - t_of(i - 2));
             bool cand = false;
             double tu = 0.0;
             if (i >= 3 && dvp < a.thr && a.thr <= dv) {
@@ -182,6 +188,7 @@ template <class T> struct Detector {
         v3 = v2;
         v2 = v1;
         v1 = vi;
+        rp = rp + 1 == a.ring_len ? 0 : rp + 1;
     }
 
     // end of the trace at sample count m: the last two samples, then close every beat
