@@ -234,3 +234,39 @@ def test_restitution_classification_vs_reference_fixture(gpu, orc):
                     assert abs(got - ref) <= 1e-9, (c["name"], got, ref)
             _say("  %s: %d beats, early %s, APD90 %s DI %s" % (c["name"], cnt[i], c["early"],
                                                              apd[i], di[i]))
+
+
+@pytest.mark.parametrize("name,precision", [("TNNP_epi", "fp64"), ("TNNP_endo", "mixed"),
+                                            ("ORd", "fp64"), ("ORd", "mixed")])
+@pytest.mark.parametrize("n", [1, 64, 65, 200])
+def test_split_batch_equals_one_cell_per_lane(gpu, orc, name, precision, n):
+    """Up to 16384 cells a cell's step runs on four waves; the same cells as the first n of a
+    batch of 16385 run one per lane.  Same expressions on the same inputs, at most contracted
+    differently: 1e-12 (FP64) and 2e-5 (FP32, 300 steps of a few 6e-8 roundings) relative, and
+    the same beats; run lengths that end inside and at the end of a chunk, and of 0 steps."""
+    _say("split batch", name, precision, n)
+    _, _, key, word, amp = MODELS[name]
+    big, steps = 16385, 300
+    rng = np.random.default_rng(n)
+    lens = rng.integers(1, steps + 1, big)
+    lens[:3] = [steps, 0, 128]
+    arrays = (rng.uniform(0.0, 1.0, big), rng.uniform(280, 400, big), rng.uniform(0.8, 1.2, big),
+              amp * rng.uniform(0.95, 1.1, big))
+    scale = rng.uniform(0.7, 1.3, (4, big))
+    out = []
+    for m in (n, big):
+        ion = gpu.IonicModel(key, word, m, solve_vm=True, precision=precision)
+        ion.set_protocol_arrays(*(a[:m] for a in arrays), 2, 250.0, 1)
+        ion.set_run_lengths(lens[:m])
+        ion.set_conductance_scale(scale[:, :m])
+        ion.enable_beats(max_beats=4, dvdt_threshold=THR, baseline_s=BASE_MS * 1e-3,
+                         peak_window_s=PEAK_MS * 1e-3)
+        gpu.batch_run([ion], DT_MS * 1e-3, chunk=128)
+        counts, rec = ion.beats()
+        out.append((ion.states()[:, :n], counts[:n], rec[:n]))
+    (s0, c0, r0), (s1, c1, r1) = out
+    tol = 1e-12 if precision == "fp64" else 2e-5
+    np.testing.assert_allclose(s0, s1, rtol=tol, atol=1e-15 if precision == "fp64" else 1e-9)
+    np.testing.assert_array_equal(c0, c1)
+    np.testing.assert_array_equal(np.isnan(r0), np.isnan(r1))
+    np.testing.assert_allclose(np.nan_to_num(r0), np.nan_to_num(r1), rtol=tol, atol=1e-9)
