@@ -30,6 +30,7 @@
 #include <hip/hip_runtime.h>
 
 #include "cg_general.hpp"
+#include "cg_hexops.hpp"
 #include "cg_reduce.hpp"
 
 namespace cg {
@@ -64,7 +65,7 @@ struct GView {
 __global__ __launch_bounds__(GBS) void k_ggrad(GView g, const double* __restrict__ V,
                                                double* __restrict__ grad)
 {
-    const int64_t c = (int64_t)blockIdx.x * GBS + threadIdx.x;
+    const int64_t c = (int64_t)xcd_block(blockIdx.x, gridDim.x) * GBS + threadIdx.x;
     if (c >= g.n) return;
     const double vp = V[c];
     double sx = 0.0, sy = 0.0, sz = 0.0;
@@ -162,7 +163,7 @@ __global__ __launch_bounds__(GBS) void k_gexplicit(GView g, const double* __rest
                                                    uint8_t* __restrict__ flag,
                                                    double* __restrict__ tact, GeneralStep st)
 {
-    const int64_t c = (int64_t)blockIdx.x * GBS + threadIdx.x;
+    const int64_t c = (int64_t)xcd_block(blockIdx.x, gridDim.x) * GBS + threadIdx.x;
     if (c >= g.n) return;
     const double vn = V[c];
     const double lap = flux_sum(g, V, grad, c, vn, true) / g.vol[c];
@@ -220,8 +221,10 @@ __global__ __launch_bounds__(RBS) void k_grhs(GView g, const double* __restrict_
                                               GeneralStep st)
 {
     double v[1] = {0.0};
-    for (int64_t c = (int64_t)blockIdx.x * RBS + threadIdx.x; c < g.n;
-         c += (int64_t)gridDim.x * RBS) {
+    const int64_t chunk = ((g.n + gridDim.x - 1) / gridDim.x + RBS - 1) / RBS * RBS;
+    const int64_t lo = (int64_t)xcd_block(blockIdx.x, gridDim.x) * chunk;
+    const int64_t hi = lo + chunk < g.n ? lo + chunk : g.n;
+    for (int64_t c = lo + threadIdx.x; c < hi; c += RBS) {
         const double vn = Vn[c];
         const double vo = st.c00 != 0.0 || extrapolate ? Vm1[c] : 0.0;
         const double src = st.src ? st.src[c] : general_box(g, c, st.boxes);
@@ -615,7 +618,8 @@ const int32_t* general_owner(const GeneralMesh* G) { return G->owner.data(); }
 const int32_t* general_neighbour(const GeneralMesh* G) { return G->nbr.data(); }
 int64_t general_faces(const GeneralMesh* G) { return G->F; }
 
-static unsigned grid_of(int64_t n) { return (unsigned)((n + GBS - 1) / GBS); }
+// (a multiple of 8: each XCD takes a contiguous eighth of the cells)
+static unsigned grid_of(int64_t n) { return (unsigned)(((n + GBS - 1) / GBS + 7) / 8 * 8); }
 
 hipError_t general_laplacian(GeneralMesh* G, const double* V, double* lap, hipStream_t s)
 {

@@ -25,6 +25,7 @@
 #include <string>
 #include <vector>
 #include "cg_ldu.hpp"
+#include "cg_hexops.hpp"
 #include "cg_reduce.hpp"
 
 namespace cg {
@@ -75,10 +76,11 @@ CG_DEV double ell_rowsum(const EllView& E, int64_t i)
     return a;
 }
 
-// contiguous chunk of rows per block for the reducing kernels
+// contiguous chunk of rows per block for the reducing kernels, each XCD a contiguous eighth
+// (its rows, and most of what they gather, stay in its own L2 from one kernel to the next)
 #define ROW_LOOP(N)                                                                        \
     const int64_t chunk_ = (((N) + gridDim.x - 1) / gridDim.x + RBS - 1) / RBS * RBS;      \
-    const int64_t lo_ = (int64_t)blockIdx.x * chunk_;                                      \
+    const int64_t lo_ = (int64_t)xcd_block(blockIdx.x, gridDim.x) * chunk_;                \
     const int64_t hi_ = lo_ + chunk_ < (N) ? lo_ + chunk_ : (N);                           \
     for (int64_t i = lo_ + threadIdx.x; i < hi_; i += RBS)
 
