@@ -51,26 +51,22 @@ def algo_bytes_per_cell(kernel, prec, model, algorithm, od_planes=1):
     s = NSTATES[model] - 1
     if kernel == "ionic":
         if algorithm == "implicit":
-            # V^n read, states r/w, Iion + rhs written; V^{n-1} and the activation flag
-            # read for the previous step's activation update; mixed: the extrapolated
-            # initial guess written as well
-            return 8 + 2 * s * w + 8 + 8 + 8 + 1 + (8 if prec == "mixed" else 0)
-        return 8 + 2 * s * w + 8 + 8 + 1  # V^n, states, Iion, V^{n+1}, flag
+            # V^n read, states r/w, rhs and the extrapolated initial guess written; V^{n-1}
+            # and the activation flag read for the previous step's activation update (Iion
+            # is stored by a call's last step only)
+            return 8 + 2 * s * w + 8 + 8 + 1 + 8
+        return 8 + 2 * s * w + 8 + 1  # V^n, states, V^{n+1}, flag
     if kernel == "spmv_dot":         # u, 3 face coefficients read; w written
         return 5 * w
     if kernel == "cg_update":        # u, p, w, s, r, 1/diag, x read; p, s, x, r, u written
         return 12 * w
-    if kernel == "residual_first":
-        # b, 3 fp64 coefficients, 1/diag, x0 read; r, u written; plus
-        #   fp64: x0 = V^n copied into V^{n+1};
-        #   mixed: x0 (written by the ionic kernel) and V^n for the correction;
-        #   correction: od planes read, corrected b written (mixed; fp64 keeps it in r)
-        base = 8 + 24 + w + 8 + 2 * w
-        if prec == "fp64":
-            return base + 8 + 8 * od_planes
-        return base + 8 * od_planes + (8 + 8 if od_planes else 0)
-    if kernel == "residual":         # x, e, b, 3 fp64 coefficients, 1/diag; x', r, u written
-        return 8 + 4 + 8 + 24 + 4 + 8 + 2 * 4
+    # conductivities constant per z-plane: the face coefficients are three numbers a plane
+    if kernel == "residual_first":   # x0, b read; r, u written; correction: V^n read, b written
+        return 8 + 8 + 2 * w + (8 + 8 if od_planes else 0)
+    if kernel == "residual":         # x, e, b read; x', r, u written
+        return 8 + 4 + 8 + 8 + 2 * 4
+    if kernel == "chebyshev":        # x_k, x_{k-1}, b read; x_{k+1} written
+        return 4 * w
     if kernel == "activation":       # solution, flag read (V^n on crossing only)
         return 8 + 1
     return None
@@ -102,7 +98,8 @@ def kernel_symbol(kernel, prec, model, algorithm):
     t = "float" if prec == "mixed" else "double"
     if kernel == "ionic":
         if algorithm == "implicit":
-            return "cg::k_ionic_rhs<cg::%s, %s, 0>" % (model, t)  # Rush-Larsen
+            return "cg::k_ionic_rhs<cg::%s, %s, 0>" % (
+                model, t if prec == "mixed" else "cg::F64")  # Rush-Larsen
         return None
     # the workload's kernels: quads (nx % 4 == 0), relative L2 norm
     return {"spmv_dot": "cg::k_cg_s<%s, true, 0>" % t,
