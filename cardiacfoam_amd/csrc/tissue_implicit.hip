@@ -923,6 +923,7 @@ struct ImplicitSolver {
     int64_t total_iters = 0;
     double last_res = 0.0;
     int last_inner = 16;
+    int prev_inner = 16;     // FP64 CG: the iterations of the solve before
     long long iters_sum_seen = 0;  // DevState::iters_sum at the previous read
     SolveControls ctl;
     double* bc = nullptr;    // b plus the correction of the current outer corrector (mixed)
@@ -1454,7 +1455,11 @@ int implicit_step(ImplicitSolver* S, int model, int prec, int tissue, void* stat
                         started ? nullptr : S->od, A, S->b, nullptr, 1);
             cg.s_kernel(gen, 0, tol * tol, 0, 0.0, 0.0, max_iter, tol, 1);
             int k = 0;
-            int chunk = S->last_inner + 1 > 2 ? S->last_inner + 1 : 2;
+            // as many iterations as either of the last two solves took: a launch beyond the
+            // end costs the host as much as one that works (a 4305-cell step is bound by its
+            // 15 launches; 13 without a spare iteration), a missing one a read-back
+            int chunk = S->last_inner > S->prev_inner ? S->last_inner : S->prev_inner;
+            chunk = chunk > 1 ? chunk : 1;
             for (;;) {
                 for (int q = 0; q < chunk; ++q, ++k) {
                     cg.u_kernel(gen, k, Vnew, 0);
@@ -1475,6 +1480,7 @@ int implicit_step(ImplicitSolver* S, int model, int prec, int tissue, void* stat
                         prof->resolve(false);
                     }
                     used_total += h.iters;
+                    S->prev_inner = S->last_inner;
                     S->last_inner = h.iters > 0 ? h.iters : S->last_inner;
                     const double bb = h.s[S_BB] > 0 ? h.s[S_BB] : 1.0;
                     S->last_res = of ? h.l1 / h.nf : std::sqrt(h.s[S_RR] / bb);
@@ -1491,7 +1497,7 @@ int implicit_step(ImplicitSolver* S, int model, int prec, int tissue, void* stat
                     *err = "solver state read-back did not report the end of the solve";
                     return 4;
                 }
-                chunk = 4;  // not finished: continue the same solve
+                chunk = 2;  // not finished: continue the same solve
             }
             log.clear();
             ++solves;
