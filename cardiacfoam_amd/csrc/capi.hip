@@ -1043,9 +1043,8 @@ static hipError_t download_planes(const void* dev, bool f32, int64_t n, int nv,
                                   const double* refs, double* host)
 {
     constexpr int64_t PIECE = 512 * 1024;
-    const int64_t per_plane = f32 ? (n + PIECE - 1) / PIECE : 0;
     const int64_t total = n * nv;
-    const int64_t pieces = f32 ? per_plane * nv : (total + PIECE - 1) / PIECE;
+    const int64_t pieces = (total + PIECE - 1) / PIECE;   // across planes
     std::atomic<int64_t> next{0};
     std::atomic<int> err{(int)hipSuccess};
     int device = 0;
@@ -1053,7 +1052,7 @@ static hipError_t download_planes(const void* dev, bool f32, int64_t n, int nv,
     auto work = [&](bool other) {
         if (other && hipSetDevice(device) != hipSuccess) return;   // the caller does the rest
         std::unique_ptr<float[]> f;
-        if (f32) f.reset(new (std::nothrow) float[(size_t)(n < PIECE ? n : PIECE)]);
+        if (f32) f.reset(new (std::nothrow) float[(size_t)(total < PIECE ? total : PIECE)]);
         if (f32 && !f) {
             err = (int)hipErrorOutOfMemory;
             return;
@@ -1062,17 +1061,17 @@ static hipError_t download_planes(const void* dev, bool f32, int64_t n, int nv,
             const int64_t q = next.fetch_add(1);
             if (q >= pieces || err.load() != (int)hipSuccess) return;
             hipError_t e;
+            const int64_t at = q * PIECE, m = total - at < PIECE ? total - at : PIECE;
             if (f32) {
-                const int64_t v = q / per_plane, i0 = q % per_plane * PIECE;
-                const int64_t m = n - i0 < PIECE ? n - i0 : PIECE;
-                const int64_t at = v * n + i0;
                 e = hipMemcpy(f.get(), (const float*)dev + at, sizeof(float) * m,
                               hipMemcpyDeviceToHost);
-                const double ref = refs[v];
-                for (int64_t i = 0; i < m && e == hipSuccess; ++i)
-                    host[at + i] = ref + (double)f[i];
+                for (int64_t i = 0; i < m && e == hipSuccess;) {
+                    const int64_t v = (at + i) / n;           // plane, and its end here
+                    const int64_t end = (v + 1) * n - at < m ? (v + 1) * n - at : m;
+                    const double ref = refs[v];
+                    for (; i < end; ++i) host[at + i] = ref + (double)f[i];
+                }
             } else {
-                const int64_t at = q * PIECE, m = total - at < PIECE ? total - at : PIECE;
                 e = hipMemcpy(host + at, (const double*)dev + at, sizeof(double) * m,
                               hipMemcpyDeviceToHost);
             }
