@@ -83,7 +83,10 @@ CG_DEV void beat_finish(Beat& b, const BatchArgs& a, int64_t cell, int& nb)
     b.flags = 0;
 }
 
-template <class T> struct Detector {
+// RL: the Rush-Larsen kernels' detector keeps its ring position and divides without scaling.
+// The adaptive kernels keep the remainder and the plain division: with the new ones a FP64
+// RKF45 batch test ran past its time limit, for a cause not found.
+template <class T, bool RL> struct Detector {
     const BatchArgs& a;
     int64_t lane, cell;
     T* ring;
@@ -104,7 +107,7 @@ template <class T> struct Detector {
         beat_load(cur, a.det, n, lane, DS_CUR);
         beat_load(old, a.det, n, lane, DS_OLD);
         nb = a.nbeats[cell];
-        rp = (int)(a.s0 % a.ring_len);
+        if constexpr (RL) rp = (int)(a.s0 % a.ring_len);
     }
     CG_DEV void store()
     {
@@ -125,14 +128,14 @@ template <class T> struct Detector {
         bool any = false;
         vmin = __builtin_inf();
         const int64_t lo = i - a.ring_len + 1 > 0 ? i - a.ring_len + 1 : 0;
-        int r = rp;
+        int r = RL ? rp : 0;
         for (int64_t j = i; j >= lo; --j) {
             const int at = r;
-            r = r == 0 ? a.ring_len - 1 : r - 1;
+            if constexpr (RL) r = r == 0 ? a.ring_len - 1 : r - 1;
             const double tj = t_of(j);
             if (tj >= tu) continue;
             if (tj < tu - a.baseline) break;
-            const double v = (double)ring[at * a.n + lane];
+            const double v = (double)ring[(RL ? at : j % a.ring_len) * a.n + lane];
             if (v < vmin) vmin = v;
             any = true;
         }
@@ -151,9 +154,11 @@ template <class T> struct Detector {
     // sample i (value vi) after step i + 1
     CG_DEV void push(int64_t i, double vi)
     {
-        ring[rp * a.n + lane] = T(vi);
+        ring[(RL ? rp : i % a.ring_len) * a.n + lane] = T(vi);
         if (i >= 2) {
-            const double dv = div_f64(vi - v2, t_of(i) - t_of(i - 2));
+            double dv;
+            if constexpr (RL) dv = div_f64(vi - v2, t_of(i) - t_of(i - 2));
+            else dv = (vi - v2) / (t_of(i) - t_of(i - 2));
             bool cand = false;
             double tu = 0.0;
             if (i >= 3 && dvp < a.thr && a.thr <= dv) {
@@ -188,7 +193,7 @@ template <class T> struct Detector {
         v3 = v2;
         v2 = v1;
         v1 = vi;
-        rp = rp + 1 == a.ring_len ? 0 : rp + 1;
+        if constexpr (RL) rp = rp + 1 == a.ring_len ? 0 : rp + 1;
     }
 
     // end of the trace at sample count m: the last two samples, then close every beat
@@ -266,7 +271,7 @@ void k_cells_protocol(T* __restrict__ st, KParams<T> P, const T* __restrict__ gs
     T y[M::NS], sw[M::NS];
     load_model_states<M>(y, sw, st, n, cell, 0);
     const Stimulus stim = a.prot ? a.prot[cell] : a.stim;
-    Detector<T> det{a, lane, cell, (T*)a.ring};
+    Detector<T, INTEG == 0> det{a, lane, cell, (T*)a.ring};
     if (a.det) det.load();
     if constexpr (INTEG == 0) {
         for (int64_t s = a.s0; s < s1; ++s) {
@@ -403,7 +408,7 @@ __global__ __launch_bounds__(256) void k_cells_split(T* __restrict__ st, KParams
     for (int q = role; q < M::NS; q += 4) buf[0][q * 64 + lid] = st[q * n + cell];
     const Stimulus stim = a.prot ? a.prot[cell] : a.stim;
     const bool detect = role == 3 && a.det && run;
-    Detector<T> det{a, lane, cell, (T*)a.ring};
+    Detector<T, true> det{a, lane, cell, (T*)a.ring};
     if (detect) det.load();
     __syncthreads();
     int cur = 0;

@@ -346,19 +346,28 @@ __global__ __launch_bounds__(MBS) void k_explicit_hex(
     T y[M::NS], sw[M::NS];
     load_model_states<M>(y, sw, st, n, c, 1);
     const double vn = V[c];
-    // the diffusion part before the model's arithmetic, so that one wait covers the state's
-    // and the stencil's loads (a step of a small mesh is the latency of its chain)
-    double lap = hex_laplacian<UNIFORM>(V, c, ix, g, a);
-    if (s.od) lap += hex_tensor_correction(V, s.od, n, c, ix.i, ix.j, ix.k, g, s.od_mask);
-    const double vo = s.c00 != 0.0 ? Vold[c] : 0.0;
-    const uint8_t fl = flag[c];
-    const double src = box_source(ix.i, ix.j, ix.k, c, g, s.boxes);
+    double lap, vo = 0.0, src;
+    uint8_t fl;
+    auto diffusion = [&]() __attribute__((always_inline)) {
+        lap = hex_laplacian<UNIFORM>(V, c, ix, g, a);
+        if (s.od) lap += hex_tensor_correction(V, s.od, n, c, ix.i, ix.j, ix.k, g, s.od_mask);
+        if (s.c00 != 0.0) vo = Vold[c];
+        fl = flag[c];
+        src = box_source(ix.i, ix.j, ix.k, c, g, s.boxes);
+    };
+    // Models of up to four states: the diffusion part before the model's arithmetic, so that
+    // one wait covers the states' and the stencil's loads (a step of a small mesh is the
+    // latency of its chain).  Larger models: after it; its registers held across the model
+    // cost waves, which hide the loads.
+    constexpr bool early = M::NS <= 4;
+    if constexpr (early) diffusion();
     const T v = model_v<M, T>(vn);
     const T I = tissue_advance<M, T, INTEG>(v, y, sw, T(s.dt_model), p, tissue, one, s.ode, c);
     store_states(sw, st, n, c, 1);
     const double iion = double(I) * M::ISCALE;
     if (Iion) Iion[c] = iion;
 
+    if constexpr (!early) diffusion();
     double rhs = s.c0 * vn + div_f64(s.dt, s.chiCm) * (lap - s.chiCm * iion + src);
     if (s.c00 != 0.0) rhs -= s.c00 * vo;
     const double vnew = div_f64(rhs, s.c);
