@@ -51,18 +51,20 @@ def algo_bytes_per_cell(kernel, prec, model, algorithm, od_planes=1):
     s = NSTATES[model] - 1
     if kernel == "ionic":
         if algorithm == "implicit":
-            # V^n read, states r/w, rhs and the extrapolated initial guess written; V^{n-1}
-            # and the activation flag read for the previous step's activation update (Iion
-            # is stored by a call's last step only)
-            return 8 + 2 * s * w + 8 + 8 + 1 + 8
+            # V^n read, states r/w, rhs written; V^{n-1} and the activation flag read for the
+            # previous step's activation update (Iion is stored by a call's last step only);
+            # mixed: the extrapolated initial guess written as well
+            return 8 + 2 * s * w + 8 + 8 + 1 + (8 if prec == "mixed" else 0)
         return 8 + 2 * s * w + 8 + 1  # V^n, states, V^{n+1}, flag
     if kernel == "spmv_dot":         # u, 3 face coefficients read; w written
         return 5 * w
     if kernel == "cg_update":        # u, p, w, s, r, 1/diag, x read; p, s, x, r, u written
         return 12 * w
     # conductivities constant per z-plane: the face coefficients are three numbers a plane
-    if kernel == "residual_first":   # x0, b read; r, u written; correction: V^n read, b written
-        return 8 + 8 + 2 * w + (8 + 8 if od_planes else 0)
+    if kernel == "residual_first":
+        # x0, b read; r, u written; FP64: x0 = V^n copied into V^{n+1}; mixed with a
+        # correction: V^n read and the corrected b written
+        return 8 + 8 + 2 * w + (8 if prec == "fp64" else (8 + 8 if od_planes else 0))
     if kernel == "residual":         # x, e, b read; x', r, u written
         return 8 + 4 + 8 + 8 + 2 * 4
     if kernel == "chebyshev":        # x_k, x_{k-1}, b read; x_{k+1} written

@@ -16,7 +16,7 @@
 //   fp64 path : CG in fp64 to ||b - A x||_2 <= tol ||b||_2.
 //   mixed path: iterative refinement; residual and solution in fp64, each correction from
 //               an fp32 CG (fp32 operator and vectors, fp64 dot products) to 1e-4 relative.
-// Where the matrix is diagonally dominant enough (below) both paths take Chebyshev's
+// Where the matrix is diagonally dominant enough (below) the mixed path takes Chebyshev's
 // iteration in place of the conjugate gradients; see k_cheb.
 // Kernels of one CG step:
 //   residual (first)  x0 = V^n, b += tensor correction, r = b - A x0, u = M^-1 r
@@ -40,7 +40,6 @@
 namespace cg {
 
 constexpr int BS = 256;    // elementwise kernels
-constexpr int SMALL_N = 8192;  // most cells of an FP64 solve that stays with the CG
 
 // partial-sum slots (RG doubles each)
 enum { P_G = 0,      // (r,u), parity sets 0 and 1
@@ -51,7 +50,7 @@ enum { P_G = 0,      // (r,u), parity sets 0 and 1
        P_L1 = 7,     // sum |r| (OpenFOAM norm), parity sets 7 and 8
        P_NF = 9,     // normalisation factor terms of the solve's first residual
        P_XS = 10,    // sum of the initial guess (its mean is OpenFOAM's xRef)
-       P_RRI = 11,   // (r,r) of a Chebyshev solve's first residual (FP64 path)
+       P_RRI = 11,   // (r,r) of a Chebyshev solve's first residual
        P_NSLOT = 12 };
 
 enum { S_RR, S_BB, S_R0, S_NSCAL };
@@ -692,66 +691,43 @@ __global__ __launch_bounds__(RBS) void k_cg_u(HexGeom g, const T* __restrict__ i
 // after k steps the error (in the norm of D) is at most 2 sigma^k / (1 + sigma^2k) of the
 // first, sigma = rho / (1 + sqrt(1 - rho^2)).  No step needs a dot product, so an iteration
 // is one kernel that reads x_k, x_{k-1}, b and the face coefficients and writes x_{k+1}
-// over x_{k-1}: 16 B per cell FP32 (layered) where the two CG kernels move 56 B and wait
-// for a grid-wide sum each.  At 2.1M cells (rho 0.13) a step takes 7.3 us FP32 and 13.1 us
-// FP64 where a CG iteration took 20.8 and 41.7 us, and the mixed solve's residual passes
-// 22 us with layered coefficients instead of 34 us.
+// over x_{k-1}: 16 B per cell (layered) where the two CG kernels move 56 B and wait for a
+// grid-wide sum each.  At 2.1M cells (rho 0.13) a step takes 7.3 us where a CG iteration took
+// 20.8 us, and the solve's residual passes 22 us with layered coefficients instead of 34 us.
+// For the corrections of the mixed path only: an FP64 solve keeps the conjugate gradients
+// from V^n.  Both stop below the tolerance, but at different points within it (1e-7 V apart
+// at 1e-8), and where a model switches on its potential (BuenoOrovio's Heavisides, Stewart's
+// and Courtemanche's branches) or a cell is about to activate, that much decides: an FP64
+// run's outputs moved by up to 1e-2.
 //
-// One step of x (k_cheb): out = xm + omega (x - xm + (b - A x)/diag), xm null: 0 (the first
-// step, w_1 = 1, needs none).  out may be xm itself.
-//   CORR (first step of a solve, FP64): b += tensor correction of vcor, written back.
-//   NORMS: partial sums |b - A x|^2 -> slot rr_slot, |b|^2 -> P_BB.
-template <class T, bool QUAD, bool LAY, bool CORR, bool NORMS>
-__global__ __launch_bounds__(RBS) void k_cheb(HexGeom g, HexOp<T> A, Layers<T> L, T omega,
-                                              const T* __restrict__ x, const T* xm, T* out,
-                                              T* b, const double* __restrict__ vcor,
-                                              const double* __restrict__ od, unsigned od_mask,
-                                              double* __restrict__ part, int rr_slot)
+// One step of x (k_cheb): out = xm + omega (x - xm + (b - A x)/diag), xm null: 0.  out may be
+// xm itself.
+template <bool QUAD, bool LAY>
+__global__ __launch_bounds__(RBS) void k_cheb(HexGeom g, HexOp<float> A, Layers<float> L,
+                                              float omega, const float* __restrict__ x,
+                                              const float* xm, float* out,
+                                              const float* __restrict__ b)
 {
-    double v[2] = {0.0, 0.0};
     const uint32_t bid = xcd_block(blockIdx.x, gridDim.x);
-    const PlainLoad<T> X{x};
+    const PlainLoad<float> X{x};
     if constexpr (QUAD) {
         RANGE_LOOP_Q(g)
         {
             const int64_t c0 = qi * 4;
             const IJK q = ijk_of((uint32_t)c0, g);
-            V4<T> bc = ld4(b + c0), xc, d;
-            const V4<T> xo = xm ? ld4(xm + c0) : V4<T>(T(0));
-            if constexpr (CORR) {
-                bc += quad_correction_xy<LAY>(vcor, LAY ? L.od : od, c0, q, g);
-                st4(b + c0, bc);
-            }
-            const V4<T> r = bc - apply_quad_diag<T, LAY>(A, L, X, c0, q, g, xc, d);
-            st4(out + c0, xo + omega * ((xc - xo) + jacobi4<T>(r, d)));
-            if constexpr (NORMS) {
-                v[0] += dot4(r, r);
-                v[1] += dot4(bc, bc);
-            }
+            V4<float> xc, d;
+            const V4<float> bc = ld4(b + c0), xo = xm ? ld4(xm + c0) : V4<float>(0.0f);
+            const V4<float> r = bc - apply_quad_diag<float, LAY>(A, L, X, c0, q, g, xc, d);
+            st4(out + c0, xo + omega * ((xc - xo) + jacobi4<float>(r, d)));
         }
     } else {
         RANGE_LOOP_B(g)
         {
             const IJK q = ijk_of((uint32_t)c, g);
-            T bc = b[c], xc, d;
-            const T xo = xm ? xm[c] : T(0);
-            if constexpr (CORR) {
-                bc += hex_tensor_correction(vcor, od, n, c, q.i, q.j, q.k, g, od_mask);
-                b[c] = bc;
-            }
-            const T r = bc - apply_row_diag<T, LAY>(A, L, X, c, q, g, xc, d);
+            float xc, d;
+            const float xo = xm ? xm[c] : 0.0f;
+            const float r = b[c] - apply_row_diag<float, LAY>(A, L, X, c, q, g, xc, d);
             out[c] = xo + omega * ((xc - xo) + jacobi(r, d));
-            if constexpr (NORMS) {
-                v[0] += double(r) * double(r);
-                v[1] += double(bc) * double(bc);
-            }
-        }
-    }
-    if constexpr (NORMS) {
-        block_sum<RBS, 2>(v);
-        if (threadIdx.x == 0) {
-            part[rr_slot * RG + bid] = v[0];
-            part[P_BB * RG + bid] = v[1];
         }
     }
 }
@@ -913,11 +889,8 @@ struct ImplicitSolver {
     float* lay32 = nullptr;
     double smax = 0.0;       // largest sum of a row's face coefficients
     // Chebyshev: initial residuals of the last step's correctors (in the controls' norm; 0:
-    // unknown) that size the next step's iteration, and whether x0 of the next FP64 solve
-    // was written into V^{n+1} (else into xalt)
+    // unknown) that size the next step's iteration
     double last_init_res[4] = {0.0, 0.0, 0.0, 0.0};
-    bool x0_in_new = false;
-    bool next_even = false;
     bool quad = false;       // nx % 4 == 0: CG kernels on quads of cells (vector loads)
     long long gen = 0;       // generation of the last CG solve started
     int64_t total_iters = 0;
@@ -1007,7 +980,6 @@ int implicit_create(ImplicitSolver** out, const HexGeom& g, const double* sig, d
     A((void**)&S->partials, 8 * RG * P_NSLOT);
     A((void**)&S->S, sizeof(DevState));
     if (offdiag) A((void**)&S->od, 8 * 3 * n);
-    A((void**)&S->xalt, 8 * n);
     if (S->layered) {
         A((void**)&S->lay, 8 * 3 * g.nz); A((void**)&S->lay_od, 8 * g.nz);
         A((void**)&S->lay32, 4 * 3 * g.nz);
@@ -1018,6 +990,7 @@ int implicit_create(ImplicitSolver** out, const HexGeom& g, const double* sig, d
         A((void**)&S->v32.r, 4 * n); A((void**)&S->v32.u, 4 * n); A((void**)&S->v32.p, 4 * n);
         A((void**)&S->v32.s, 4 * n); A((void**)&S->v32.w, 4 * n);
         A((void**)&S->e32, 4 * n);
+        A((void**)&S->xalt, 8 * n);
     } else {
         A((void**)&S->v64.r, 8 * n); A((void**)&S->v64.u, 8 * n); A((void**)&S->v64.p, 8 * n);
         A((void**)&S->v64.s, 8 * n); A((void**)&S->v64.w, 8 * n);
@@ -1224,35 +1197,19 @@ template <class T> struct CgRun {
     }
 };
 
-// one Chebyshev step out = xm + omega (x - xm + D^-1 (b - A x)); corr: b += correction of
-// vcor first; rr_slot >= 0: with the residual's partial sums
-template <class T>
-void cheb_step(ImplicitSolver* S, Profiler* prof, const HexOp<T>& A, double omega, const T* x,
-               const T* xm, T* out, T* b, const double* vcor, bool corr, int rr_slot)
+// one Chebyshev step out = xm + omega (x - xm + D^-1 (b - A x))
+void cheb_step(ImplicitSolver* S, Profiler* prof, const HexOp<float>& A, double omega,
+               const float* x, const float* xm, float* out, const float* b)
 {
     const int tk = prof ? prof->begin(K_CHEB) : -1;
-    // quads need nx % 4 == 0 and no correction beyond sigma_xy
-    const bool quad = S->quad && (!corr || S->od_mask == 1u);
-    const Layers<T> L = layers_of<T>(S);
-#define CG_C(Q, LAY, CO, NO)                                                               \
-    hipLaunchKernelGGL((k_cheb<T, Q, LAY, CO, NO>), dim3(S->rgrid), dim3(RBS), 0, S->stream, \
-                       S->g, A, L, T(omega), x, xm, out, b, vcor, (const double*)S->od,    \
-                       S->od_mask, S->partials, rr_slot)
-#define CG_CQ(CO, NO)                                                                      \
-    do {                                                                                   \
-        if (quad && S->layered) CG_C(true, true, CO, NO);                                  \
-        else if (quad) CG_C(true, false, CO, NO);                                          \
-        else if (S->layered) CG_C(false, true, CO, NO);                                    \
-        else CG_C(false, false, CO, NO);                                                   \
-    } while (0)
-    if constexpr (sizeof(T) == 8) {
-        if (corr) CG_CQ(true, true);
-        else if (rr_slot >= 0) CG_CQ(false, true);
-        else CG_CQ(false, false);
-    } else {
-        CG_CQ(false, false);
-    }
-#undef CG_CQ
+    const Layers<float> L = layers_of<float>(S);
+#define CG_C(Q, LAY)                                                                       \
+    hipLaunchKernelGGL((k_cheb<Q, LAY>), dim3(S->rgrid), dim3(RBS), 0, S->stream, S->g, A, L, \
+                       float(omega), x, xm, out, b)
+    if (S->quad && S->layered) CG_C(true, true);
+    else if (S->quad) CG_C(true, false);
+    else if (S->layered) CG_C(false, true);
+    else CG_C(false, false);
 #undef CG_C
     if (prof) prof->end(tk);
 }
@@ -1291,27 +1248,16 @@ int implicit_step(ImplicitSolver* S, int model, int prec, int tissue, void* stat
     // Outer correctors keep the extrapolation in the residual.
     const bool fuse = S->ctl.n_outer <= 1;
     const double* od_res = S->od;
-    // Chebyshev's iteration where rho <= 0.6: there it needs at most about one step in four
-    // more than the conjugate gradients (whose count the bound also limits), each a third of
-    // their time, and one Jacobi step never enlarges a residual (rho sqrt(dmax/dmin) < 1 as
-    // dmax/dmin <= 1/(1 - rho)).  Not for OpenFOAM's norm in FP64, whose solves the PIMPLE
-    // loop counts, nor for tolerances at the rounding of the true residual it tests, nor
-    // when few iterations are allowed, nor in FP64 up to SMALL_N cells, where a solve is
-    // launches and waits whichever iteration it runs.
-    auto rho_of = [&](double c) { return S->smax / (c * S->chiCm / S->dt + S->smax); };
-    auto use_cheb = [&](double c) {
-        return rho_of(c) <= 0.6 && max_iter >= 100 &&
-               (prec == 1 || (S->ctl.norm == 0 && fuse && tol >= 1e-13 && S->n > SMALL_N));
-    };
-    const double rho = rho_of(st.c);
-    const bool cheb = use_cheb(st.c);
-    const bool x0_fused = fuse && extrapolate && (prec == 1 || cheb);
+    // Chebyshev's iteration (mixed path) where rho <= 0.6: there it needs at most about one
+    // step in four more than the conjugate gradients (whose count the bound also limits), each
+    // a third of their time.  Not when few iterations are allowed.
+    const double rho = S->smax / (st.c * S->chiCm / S->dt + S->smax);
+    const bool cheb = prec == 1 && rho <= 0.6 && max_iter >= 100;
+    const bool x0_fused = fuse && prec == 1 && extrapolate;
     if (!ionic_queued) {
-        S->x0_in_new = prec == 0 && S->next_even;
         tk = prof ? prof->begin(K_IONIC) : -1;
         e = launch_ionic_rhs(model, prec, tissue, S->g, states, Vn, Vm1,
-                             x0_fused ? (S->x0_in_new ? Vnew : S->xalt) : nullptr, Iion, S->b,
-                             st, P, S->stream);
+                             x0_fused ? S->xalt : nullptr, Iion, S->b, st, P, S->stream);
         if (prof) prof->end(tk);
         if (e != hipSuccess) { *err = std::string("ionic/rhs launch: ") + hipGetErrorString(e); return 4; }
     }
@@ -1365,12 +1311,9 @@ int implicit_step(ImplicitSolver* S, int model, int prec, int tissue, void* stat
                 sn.act_v = st.act_v;
             }
             int t = prof ? prof->begin(K_IONIC) : -1;
-            // (the next step's V^{n+1} is this one's V^{n-1}, whose last reader is done)
-            S->x0_in_new = prec == 0 && S->next_even;
-            double* x0 = !fuse || !(prec == 1 || use_cheb(sn.c)) ? nullptr
-                         : S->x0_in_new ? const_cast<double*>(Vm1) : S->xalt;
-            launch_ionic_rhs(model, prec, tissue, S->g, states, Vnew, Vn, x0, next->Iion, S->b,
-                             sn, P, S->stream);
+            launch_ionic_rhs(model, prec, tissue, S->g, states, Vnew, Vn,
+                             fuse && prec == 1 ? S->xalt : nullptr, next->Iion, S->b, sn, P,
+                             S->stream);
             if (prof) prof->end(t);
         }
         if (hipGetLastError() != hipSuccess) return false;
@@ -1384,75 +1327,15 @@ int implicit_step(ImplicitSolver* S, int model, int prec, int tissue, void* stat
     int solves = 0;
     if (prec == 0) {
         CgRun<double> cg{S, A, S->v64, prof, &log};
-        // Chebyshev from x0 = 2 V^n - V^{n-1} (V^n on the first step): a Jacobi step from x0,
-        // the iteration, a last Jacobi step whose kernel tests the residual of the iterate
-        // before it.  A pass that misses the tolerance is repeated from its result, with the
-        // steps its own residual asks for; after three the conjugate gradients take over.
-        bool started = false;      // V^{n+1} holds an iterate, b the correction
-        for (int pass = 0; cheb && pass < 3; ++pass) {
-            const long long gen = ++S->gen;
-            const double r0 = pass == 0 ? S->last_init_res[0] : S->last_res;
-            double need = r0 > 0.0 ? 0.5 * tol / r0 : 1e-5;
-            need = need < 0.3 ? need : 0.3;
-            int J = cheb_steps(rho, need) + 1;
-            const double* x = pass > 0 ? Vnew : x0_fused ? (S->x0_in_new ? Vnew : S->xalt) : Vn;
-            // x_J lands in V^{n+1}
-            if (x == Vnew) J += J & 1;
-            else if (x == S->xalt) J += !(J & 1);
-            const double* xm = nullptr;
-            double w = 1.0;
-            for (int j = 0; j < J; ++j) {
-                double* out = ((J - j) & 1) ? Vnew : S->xalt;
-                const bool ends = j == 0 || j == J - 1;
-                if (j == 1) w = 1.0 / (1.0 - 0.5 * rho * rho);
-                else if (j > 1) w = 1.0 / (1.0 - 0.25 * rho * rho * w);
-                cheb_step<double>(S, prof, A, ends ? 1.0 : w, x, ends ? nullptr : xm, out, S->b,
-                                  Vn, j == 0 && pass == 0 && od_res,
-                                  j == 0 ? P_RRI : j == J - 1 ? P_RR0 : -1);
-                xm = x;
-                x = out;
-            }
-            started = true;
-            S->next_even = !(J & 1);
-            hipLaunchKernelGGL(k_cheb_check, dim3(1), dim3(RG), 0, S->stream,
-                               (const double*)S->partials, (int)S->rgrid, S->S, S->hS_dev, gen,
-                               0, tol, P_RR0, P_RR0, pass == 0 ? P_RRI : -1, -1);
-            size_t gated;
-            if (!finish_and_read(gen, Vnew, &gated, true)) {
-                *err = "Chebyshev launch or read-back failed";
-                return 4;
-            }
-            const DevState& h = *S->hS;
-            const bool ok = h.conv_gen == gen;
-            if (prof) {
-                if (!ok) prof->invalidate_range(gated, prof->mark());
-                prof->resolve(false);
-            }
-            used_total += J;
-            S->last_res = std::sqrt(h.s[S_RR] / (h.s[S_BB] > 0 ? h.s[S_BB] : 1.0));
-            if (pass == 0) {
-                prev_init = h.init_res;
-                S->last_init_res[0] = prev_init;
-            }
-            if (ok) {
-                S->last_solves = 1;
-                S->last_init = prev_init;
-                S->last_final = S->last_res;
-                S->total_iters += used_total;
-                return 0;
-            }
-            if (!std::isfinite(S->last_res)) break;
-        }
         // fp64 CG per corrector; x0 = V^n (copied into V^{n+1} by the first residual)
         for (int outer = 1;; ++outer) {
             const bool last = n_outer == 1 || outer >= n_outer ||
                               (outer > 1 && prev_init < S->ctl.residual_control);
             const long long gen = ++S->gen;
-            const bool from_vn = outer == 1 && !started;
-            const double* xin = from_vn ? Vn : Vnew;
+            const double* xin = outer == 1 ? Vn : Vnew;
             if (of) cg.mean(xin, nullptr);
-            cg.residual(K_RESIDUAL0, gen, xin, nullptr, nullptr, from_vn ? Vnew : nullptr,
-                        started ? nullptr : S->od, A, S->b, nullptr, 1);
+            cg.residual(K_RESIDUAL0, gen, xin, nullptr, nullptr, outer == 1 ? Vnew : nullptr,
+                        outer == 1 ? od_res : S->od, A, S->b, nullptr, 1);
             cg.s_kernel(gen, 0, tol * tol, 0, 0.0, 0.0, max_iter, tol, 1);
             int k = 0;
             // as many iterations as either of the last two solves took: a launch beyond the
@@ -1485,7 +1368,6 @@ int implicit_step(ImplicitSolver* S, int model, int prec, int tissue, void* stat
                     const double bb = h.s[S_BB] > 0 ? h.s[S_BB] : 1.0;
                     S->last_res = of ? h.l1 / h.nf : std::sqrt(h.s[S_RR] / bb);
                     prev_init = h.init_res;
-                    if (S->last_init_res[0] == 0.0) S->last_init_res[0] = prev_init;
                     if (!ok) {
                         *err = "PCG did not converge within max_iter";
                         return 7;
@@ -1558,8 +1440,8 @@ int implicit_step(ImplicitSolver* S, int model, int prec, int tissue, void* stat
                     for (int j = 1; j < K; ++j) {
                         w = j == 1 ? 1.0 / (1.0 - 0.5 * rho * rho)
                                    : 1.0 / (1.0 - 0.25 * rho * rho * w);
-                        cheb_step<float>(S, prof, cg.A, w, eb[ei], j == 1 ? nullptr : eb[ei ^ 1],
-                                         eb[ei ^ 1], S->v32.r, nullptr, false, -1);
+                        cheb_step(S, prof, cg.A, w, eb[ei], j == 1 ? nullptr : eb[ei ^ 1],
+                                  eb[ei ^ 1], S->v32.r);
                         ei ^= 1;
                     }
                     double* nxt = cur == Vnew ? S->xalt : Vnew;

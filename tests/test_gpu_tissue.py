@@ -275,10 +275,10 @@ def test_activation_threshold(gpu, orc, algorithm):
 @pytest.mark.parametrize("shape", [(16, 8, 6), (13, 7, 5), (8, 1, 1), (4, 5, 1), (1, 1, 9),
                                    (260, 9, 5), (101, 12, 8)])
 def test_implicit_solver_branches(gpu, orc, shape, kind, h):
-    """Chebyshev's iteration (h = 0.2 and 0.07 mm: rho 0.13 and 0.55) and the conjugate
-    gradients (0.04 mm: rho 0.79), quads and single cells, coefficients per plane and per
-    cell (with all off-diagonal conductivities), one cell thick, on both sides of the 8192
-    cells up to which FP64 stays with the conjugate gradients: the oracle's solution.
+    """FP64's conjugate gradients, mixed: Chebyshev's iteration (h = 0.2 and 0.07 mm: rho 0.13
+    and 0.55) and the conjugate gradients (0.04 mm: rho 0.79); quads and single cells,
+    coefficients per plane and per cell (with all off-diagonal conductivities), one cell
+    thick, from one block of the reducing kernels to several: the oracle's solution.
     FP64: both solve to 1e-12 of b, whose error reaches Vm through at most 40 steps; mixed:
     FP32 gates, 40 steps of a few FP32 roundings each."""
     _say("solver branches", shape, kind, h)
@@ -302,3 +302,24 @@ def test_implicit_solver_branches(gpu, orc, shape, kind, h):
         _say("  %s: Vm rel %.2e, %d iterations, residual %.1e" % (prec, err, iters, res))
         assert res <= 1e-12 and iters > 0
         assert err <= bound
+
+
+@pytest.mark.parametrize("name,shape,ddt", [("BO_epi", (40, 24, 12), 1), ("CRN", (33, 20, 16), 0),
+                                            ("STW", (36, 20, 15), 1)])
+def test_fp64_implicit_stops_where_the_oracle_does(gpu, orc, name, shape, ddt):
+    """A solve that stops at 1e-8 leaves an error of 1e-7 of Vm, which a model's switches
+    (BuenoOrovio's Heavisides, Courtemanche's and Stewart's branches) turn into any size, so
+    the FP64 path keeps the iterates and not only the tolerance: conjugate gradients from
+    V^n, as the oracle's.  The same iterates to rounding: about 5 a step of some 30
+    roundings each, 40 steps, doubled by every mm the wave has moved; 1e-11."""
+    _say("fp64 iterates", name, shape, ddt)
+    m, tis, key, word, _ = MODELS[name]
+    h, dt, n_steps = 2e-4, 2e-5, 40
+    sig = rotating_fibre_sigma(*shape)
+    box = dict(BOX, stimulusLocationMax=[1.5e-3, 1.5e-3, 1.5e-3], stimulusIntensity=3e5)
+    T = _oracle_run(orc, shape, h, sig, m, tis, dt, n_steps, ddt, 1, box, pcg_tol=1e-8)
+    dom = gpu.Monodomain(gpu.HexMesh(*shape, h), _coeffs(key, word, "implicit", sigma=sig, box=box),
+                         dt=dt, tol=1e-8, max_iter=5000, ddt="backward" if ddt else "Euler")
+    dom.step(n_steps)
+    assert np.max(T.V) > -0.02          # the stimulated corner is past the switches
+    _compare(dom, T, vtol_rel=1e-11, ttol=1e-12)
