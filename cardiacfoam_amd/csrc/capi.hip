@@ -1549,28 +1549,33 @@ static int general_advance(cg_tissue* t, cg::GeneralMesh* G, int n_steps, bool i
                 if (!grad_ready) HIPCHK(cg::general_gradient(G, Vn, s));
                 HIPCHK(cg::general_rhs(G, Vn, Vm1, t->d_Iion, Vnew, t->d_b, ex, xs, blocks, st,
                                        s));
-                double prev = t->g_r0;   // the last step's first residual sizes this one
+                // the last step's first residual sizes this one; the target is the absolute
+                // tolerance or relTol times this solve's first residual
+                double prev = t->g_r0, target = t->g_tol;
                 for (int pass = 0; pass < 2 && !solved; ++pass) {
-                    double need = prev > 0.0 && t->g_solves > 0 ? t->g_tol / prev : 1e-5;
-                    if (need < t->g_rel) need = t->g_rel;
+                    double need = prev > 0.0 && t->g_solves > 0 ? target / prev : 1e-5;
+                    if (pass == 0 && need < t->g_rel) need = t->g_rel;
                     need = 0.5 * need < 0.3 ? 0.5 * need : 0.3;
                     t->g_iters += cg::ldu_cheb(t->gldu, s, Vnew, t->d_b, t->g_rho, need,
-                                               t->g_tol, t->g_rel);
+                                               t->g_tol, t->g_rel, pass == 0);
                     grad_ready = q + 1 < n_steps;
                     if (grad_ready) HIPCHK(cg::general_gradient(G, Vnew, s));
                     double r0, r1;
                     if (cg::ldu_cheb_wait(t->gldu, &solved, &r0, &r1))
                         return fail(CG_ERR_HIP, "Chebyshev solve failed");
-                    if (pass == 0) t->g_r0 = r0;
+                    if (pass == 0) {
+                        t->g_r0 = r0;
+                        t->g_solves = 1;
+                        if (t->g_rel * r0 > target) target = t->g_rel * r0;
+                    }
                     t->g_r1 = prev = r1;
                 }
-                t->g_solves = 1;
                 if (!solved) {
                     grad_ready = false;
                     HIPCHK(hipStreamSynchronize(s));
                     int it = 0;
                     double r0 = 0.0;
-                    if (cg::ldu_solve(t->gldu, Vnew, t->d_b, true, t->g_tol, 0.0, t->g_max_iter,
+                    if (cg::ldu_solve(t->gldu, Vnew, t->d_b, true, target, 0.0, t->g_max_iter,
                                       &it, &r0, &t->g_r1))
                         return fail(CG_ERR_HIP, "lduMatrix solve failed");
                     t->g_iters += it;

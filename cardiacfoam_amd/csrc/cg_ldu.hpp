@@ -24,10 +24,12 @@ int ldu_solve(LduSolver* L, double* psi, const double* b, bool device, double to
 // Chebyshev's iteration for a matrix whose rows, scaled by the diagonal, differ from the
 // identity by at most rho < 1 in absolute sum (the general mesh's implicit step): steps for
 // a reduction `need`, asynchronous on s from the guess in x, the solution in x, then the
-// test of OpenFOAM's norm; xs [blocks] holds the guess's partial sums (ldu_guess_sums).
+// test of OpenFOAM's norm against the solve's first residual (rel) and its normalisation,
+// which the first pass of a solve takes; xs [blocks] holds the guess's partial sums
+// (ldu_guess_sums).
 // Returns the steps; ldu_cheb_wait waits for the test and reports it.
 int ldu_cheb(LduSolver* L, hipStream_t s, double* x, const double* b, double rho, double need,
-             double tol, double rel);
+             double tol, double rel, bool first);
 int ldu_cheb_wait(LduSolver* L, bool* conv, double* init_res, double* final_res);
 // where the kernel that makes the guess puts its sums, and on how many blocks of RBS it runs
 double* ldu_guess_sums(LduSolver* L, unsigned* blocks);

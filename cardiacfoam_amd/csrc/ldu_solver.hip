@@ -412,7 +412,7 @@ double* ldu_guess_sums(LduSolver* L, unsigned* blocks)
 }
 
 int ldu_cheb(LduSolver* L, hipStream_t s, double* x, const double* b, double rho, double need,
-             double tol, double rel)
+             double tol, double rel, bool first)
 {
     const double sg = rho / (1.0 + std::sqrt(1.0 - rho * rho));
     int J = 2;
@@ -426,9 +426,10 @@ int ldu_cheb(LduSolver* L, hipStream_t s, double* x, const double* b, double rho
         double* out = ((J - j) & 1) ? x : L->u;
         if (j == 1) w = 1.0 / (1.0 - 0.5 * rho * rho);
         else if (j > 1) w = 1.0 / (1.0 - 0.25 * rho * rho * w);
-        if (j == 0)
+        // (a later pass leaves the solve's first residual and normalisation where they are)
+        if (j == 0 && first)
             hipLaunchKernelGGL((k_lcheb<true, false>), grid, blk, 0, s, E, 1.0, cur, xm, out, b, L->part);
-        else if (j == J - 1)
+        else if (j == 0 || j == J - 1)
             hipLaunchKernelGGL((k_lcheb<false, true>), grid, blk, 0, s, E, 1.0, cur, xm, out, b, L->part);
         else
             hipLaunchKernelGGL((k_lcheb<false, false>), grid, blk, 0, s, E, w, cur, xm, out, b, L->part);

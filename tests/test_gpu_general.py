@@ -236,3 +236,50 @@ def test_diffusion_step_with_caller_ionic(gpu, orc, kind, alg):
     assert (ta > 0).sum() > 0
     assert err <= (1e-12 if alg == "explicit" else 1e-9)
     assert np.array_equal(ta > 0, tb > 0) and np.max(np.abs(ta - tb)) <= 1e-10
+
+
+def _controls_run(gpu, tol, rel, max_iter, steps, iters=None):
+    """a warped block, FP64 BuenoOrovio, one solve per step; Vm and, into iters, the
+    iterations of each step"""
+    shape, L = (14, 12, 10), (2.8e-3, 2.4e-3, 2e-3)
+    m = pm.block(*shape, lengths=L, warp=pm.smooth_warp(0.05, L))
+    dom = gpu.Monodomain(_poly(gpu, m), _coeffs("implicit", rotating_fibre_sigma(*shape)),
+                         dt=2e-5, tol=1e-9, max_iter=1000)
+    dom.set_solver_controls("OpenFOAM", tol, rel, max_iter, 1, 0.0)
+    seen = 0
+    for _ in range(steps):
+        dom.step(1)
+        n = dom.solver_stats()[0]
+        if iters is not None:
+            iters.append(n - seen)
+        seen = n
+    return dom.Vm, dom.solver_report()
+
+
+def test_general_rel_tol_reaches_the_fallback(gpu, orc):
+    """Controls that rely on relTol alone, at 1e-14 of the first residual: below what a true
+    residual reaches, so both Chebyshev passes miss and the PCG, whose residual is its
+    recurrence's, ends the solve at relTol.  At most twice the 64 steps of a pass and what the
+    PCG needs by itself (fewer than 100 allowed iterations select it)."""
+    _say("general relTol")
+    with_cheb, pcg = [], []
+    V, rep = _controls_run(gpu, 1e-300, 1e-14, 1000, 6, with_cheb)
+    Vp, _ = _controls_run(gpu, 1e-300, 1e-14, 99, 6, pcg)
+    _say("  iterations a step", with_cheb, pcg, "report", rep)
+    assert max(pcg) < 99
+    assert max(with_cheb) <= 128 + 2 * max(pcg)
+    assert rep[2] <= 1e-14 * rep[1] * (1 + 1e-9)
+    assert np.max(np.abs(V - Vp)) <= 1e-12 * np.max(np.abs(Vp))
+
+
+@pytest.mark.parametrize("rel", [0.3, 1e-2, 1e-5])
+def test_general_rel_tol(gpu, orc, rel):
+    """relTol as the only criterion that binds: the solve ends below relTol times its own
+    first residual, and a looser one takes no more iterations."""
+    _say("general relTol", rel)
+    its, exact = [], []
+    V, rep = _controls_run(gpu, 1e-300, rel, 1000, 8, its)
+    _controls_run(gpu, 1e-12, 0.0, 1000, 8, exact)
+    _say("  iterations a step", its, exact, "report", rep)
+    assert rep[2] < rel * rep[1]
+    assert sum(its) <= sum(exact)
