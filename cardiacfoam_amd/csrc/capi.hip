@@ -309,6 +309,7 @@ struct cg_tissue {
     double g_r0 = 0.0, g_r1 = 0.0;
     int64_t g_iters = 0;
     double g_rho = 1.0;               // bound of the Jacobi-scaled matrix (k_cheb's rho)
+    int g_pcg_steps = 0;              // steps left that start with the PCG (see general_advance)
 };
 
 namespace {
@@ -1541,8 +1542,17 @@ static int general_advance(cg_tissue* t, cg::GeneralMesh* G, int n_steps, bool i
             // from 2 Vn - Vn-1, a second pass if the first missed, then the PCG.  While the
             // host waits for the test the next step's gradient of Vnew runs (it changes
             // nothing a repeated solve would need).
+            // Chebyshev's test is the true residual, which does not get below its rounding (a
+            // tolerance of 1e-16, or a tissue at rest, whose normalisation is rounding too);
+            // the PCG's is its recurrence's, which does.  A pass that falls short of a
+            // thirtieth of its bound's reduction (the bound's norm and the test's differ by
+            // less) has met that floor: the PCG ends the solve at once and starts the next 15,
+            // before another try.  1680 cells at rest, 1e-16: 22 to 29 iterations on such a
+            // step and 13 on the others, where every step took 45.
             bool solved = false;
-            if (t->g_outer <= 1 && t->g_rho <= 0.6 && t->g_max_iter >= 100) {
+            if (t->g_pcg_steps > 0) {
+                --t->g_pcg_steps;
+            } else if (t->g_outer <= 1 && t->g_rho <= 0.6 && t->g_max_iter >= 100) {
                 const bool ex = t->steps >= 1;
                 unsigned blocks;
                 double* xs = cg::ldu_guess_sums(t->gldu, &blocks);
@@ -1568,7 +1578,12 @@ static int general_advance(cg_tissue* t, cg::GeneralMesh* G, int n_steps, bool i
                         t->g_solves = 1;
                         if (t->g_rel * r0 > target) target = t->g_rel * r0;
                     }
+                    const bool floor = !(r1 <= 30.0 * need * (pass == 0 ? r0 : prev));
                     t->g_r1 = prev = r1;
+                    if (!solved && (floor || pass == 1)) {
+                        t->g_pcg_steps = 15;
+                        break;
+                    }
                 }
                 if (!solved) {
                     grad_ready = false;

@@ -238,13 +238,15 @@ def test_diffusion_step_with_caller_ionic(gpu, orc, kind, alg):
     assert np.array_equal(ta > 0, tb > 0) and np.max(np.abs(ta - tb)) <= 1e-10
 
 
-def _controls_run(gpu, tol, rel, max_iter, steps, iters=None):
+def _controls_run(gpu, tol, rel, max_iter, steps, iters=None, rest=False):
     """a warped block, FP64 BuenoOrovio, one solve per step; Vm and, into iters, the
-    iterations of each step"""
+    iterations of each step; rest: without the stimulus"""
     shape, L = (14, 12, 10), (2.8e-3, 2.4e-3, 2e-3)
     m = pm.block(*shape, lengths=L, warp=pm.smooth_warp(0.05, L))
-    dom = gpu.Monodomain(_poly(gpu, m), _coeffs("implicit", rotating_fibre_sigma(*shape)),
-                         dt=2e-5, tol=1e-9, max_iter=1000)
+    coeffs = _coeffs("implicit", rotating_fibre_sigma(*shape))
+    if rest:
+        coeffs["externalStimulus"] = dict(BOX, stimulusStartTime=1.0)
+    dom = gpu.Monodomain(_poly(gpu, m), coeffs, dt=2e-5, tol=1e-9, max_iter=1000)
     dom.set_solver_controls("OpenFOAM", tol, rel, max_iter, 1, 0.0)
     seen = 0
     for _ in range(steps):
@@ -283,3 +285,23 @@ def test_general_rel_tol(gpu, orc, rel):
     _say("  iterations a step", its, exact, "report", rep)
     assert rep[2] < rel * rep[1]
     assert sum(its) <= sum(exact)
+
+
+@pytest.mark.parametrize("tol", [1e-9, 1e-16])
+@pytest.mark.parametrize("rest", [False, True])
+def test_general_residual_floor(gpu, orc, tol, rest):
+    """A tolerance that the true residual cannot reach (1e-16; or any at rest, where the
+    normalisation is rounding as well) is not tried again in every step: over 32 steps two
+    tries of Chebyshev's iteration, of at most 64 steps each, beside what the PCG takes by
+    itself (fewer than 100 allowed iterations select it; from the slightly other potentials a
+    step of it may take one or two more)."""
+    _say("general floor", tol, rest)
+    its, pcg = [], []
+    run = lambda mx, out: _controls_run(gpu, tol, 0.0, mx, 32, out, rest)
+    V, rep = run(1000, its)
+    Vp, _ = run(99, pcg)
+    _say("  iterations a step", its, pcg, "report", rep)
+    assert max(pcg) < 99 and rep[2] < tol
+    if tol < 1e-15 or rest:
+        assert sum(its) <= sum(pcg) + 32 * 2 + 2 * 64
+    assert np.max(np.abs(V - Vp)) <= (1e-8 if tol == 1e-9 else 1e-12) * np.max(np.abs(Vp))
