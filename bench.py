@@ -51,10 +51,11 @@ def algo_bytes_per_cell(kernel, prec, model, algorithm, od_planes=1):
     s = NSTATES[model] - 1
     if kernel == "ionic":
         if algorithm == "implicit":
-            # V^n read, states r/w, rhs written; V^{n-1} and the activation flag read for the
-            # previous step's activation update (Iion is stored by a call's last step only);
-            # mixed: the extrapolated initial guess written as well
-            return 8 + 2 * s * w + 8 + 8 + 1 + (8 if prec == "mixed" else 0)
+            # V^n read, states r/w, Iion and rhs written; V^{n-1} and the activation flag read
+            # for the previous step's activation update; mixed: the extrapolated initial
+            # guess written as well
+            return 8 + 2 * s * w + 8 + 8 + 8 + 1 + (8 if prec == "mixed" else 0)
+        # (Iion is stored by a call's last step only)
         return 8 + 2 * s * w + 8 + 1  # V^n, states, V^{n+1}, flag
     if kernel == "spmv_dot":         # u, 3 face coefficients read; w written
         return 5 * w

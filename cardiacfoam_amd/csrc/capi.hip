@@ -1706,7 +1706,8 @@ int cg_tissue_step(cg_tissue* t, int n_steps)
         if (ode0.method) model_step_times(ion->model, t0, dt, &st.ode.t0, &st.ode.t1);
         return st;
     };
-    // Iion is read between calls only: the steps before the last do not store it
+    // Iion is read between calls only: the explicit steps before the last do not store it (an
+    // implicit step does, as its solve may end the call)
     bool ionic_queued = false;  // this step's ionic launch was queued by the previous one
     for (int s = 0; s < n_steps; ++s) {
         const double tn = t->t + dt;
@@ -1726,11 +1727,9 @@ int cg_tissue_step(cg_tissue* t, int n_steps)
             cg::NextIonic nx;
             const bool more = s + 1 < n_steps;
             if (more) nx.st = make_step(tn, t->steps + 1);
-            if (s + 2 >= n_steps) nx.Iion = t->d_Iion;
             int rc = cg::implicit_step(t->implicit, ion->model, ion->prec, ion->tissue,
-                                       ion->d_states, ion->P, Vn, Vm1, Vnew,
-                                       more ? nullptr : t->d_Iion, t->d_flag, t->d_tact, st,
-                                       t->cfg.tol, t->cfg.max_iter,
+                                       ion->d_states, ion->P, Vn, Vm1, Vnew, t->d_Iion,
+                                       t->d_flag, t->d_tact, st, t->cfg.tol, t->cfg.max_iter,
                                        prof, ionic_queued, more ? &nx : nullptr,
                                        t->steps >= 1, &g_err);
             if (rc != 0) return rc;

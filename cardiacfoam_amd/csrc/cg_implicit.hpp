@@ -16,7 +16,6 @@ void implicit_destroy(ImplicitSolver* S);
 // convergence): the step constants of that step
 struct NextIonic {
     ExplicitStep st;
-    double* Iion = nullptr;   // where its Iion goes; null: a step whose Iion nothing reads
 };
 // one step: ionic (V^n) + right-hand side (unless ionic_queued: the previous call already
 // queued it), solve for Vnew, activation update; with `next`, the next step's ionic kernel

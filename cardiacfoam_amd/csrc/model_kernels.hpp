@@ -380,7 +380,7 @@ __global__ __launch_bounds__(MBS) void k_explicit_hex(
 
 // ------------------------------------------ ionic step + implicit right-hand side
 // rhs = chiCm/dt (c0 V^n - c00 V^{n-1}) - chiCm Iion + source (the explicit tensor
-// correction is added by the solver's first residual); Iion may be null; x0 (when not null) receives the
+// correction is added by the solver's first residual); x0 (when not null) receives the
 // solver's extrapolated initial guess 2 V^n - V^{n-1}, riding on this kernel's pass over
 // V^n; with s.act_flag it also completes the previous step's activation times.  With a
 // gate (s.gate) the launch may be queued before the previous step's solve is known to have
@@ -423,7 +423,7 @@ void k_ionic_rhs(HexGeom g, T* __restrict__ st,
     const T I = tissue_advance<M, T, INTEG>(v, y, sw, T(s.dt_model), p, tissue, one, s.ode, c);
     store_states(sw, st, n, c, 1);
     const double iion = double(I) * M::ISCALE;
-    if (Iion) Iion[c] = iion;
+    Iion[c] = iion;
     const double src = box_source(cc.i, cc.j, cc.k, c, g, s.boxes);
     double rhs = div_f64(s.chiCm, s.dt) * (s.c0 * vn - s.c00 * vo) + src - s.chiCm * iion;
     b[c] = rhs;

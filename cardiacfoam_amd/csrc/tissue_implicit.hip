@@ -1312,7 +1312,7 @@ int implicit_step(ImplicitSolver* S, int model, int prec, int tissue, void* stat
             }
             int t = prof ? prof->begin(K_IONIC) : -1;
             launch_ionic_rhs(model, prec, tissue, S->g, states, Vnew, Vn,
-                             fuse && prec == 1 ? S->xalt : nullptr, next->Iion, S->b, sn, P,
+                             fuse && prec == 1 ? S->xalt : nullptr, Iion, S->b, sn, P,
                              S->stream);
             if (prof) prof->end(t);
         }

@@ -323,3 +323,37 @@ def test_fp64_implicit_stops_where_the_oracle_does(gpu, orc, name, shape, ddt):
     dom.step(n_steps)
     assert np.max(T.V) > -0.02          # the stimulated corner is past the switches
     _compare(dom, T, vtol_rel=1e-11, ttol=1e-12)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_iion_after_a_call_that_fails_part_way(gpu, orc, precision):
+    """A call of ten implicit steps whose sixth, the first with a stimulus, is given too few
+    iterations (the fewest with which the five before it converge): Iion is that of the sixth
+    step, as when the steps are taken one by one, and potential, time and states too."""
+    _say("Iion after a failure", precision)
+    _, _, key, word, _ = MODELS["BO_epi"]
+    dt = 2e-5
+    box = dict(BOX, stimulusStartTime=4.5 * dt, stimulusIntensity=1e8)
+    v0 = -0.084 + 0.02 * np.random.default_rng(3).random(12 * 9 * 6)
+
+    def run(max_iter, calls):
+        dom = gpu.Monodomain(gpu.HexMesh(12, 9, 6, 2e-4), _coeffs(key, word, "implicit", box=box),
+                             dt=dt, tol=1e-7, max_iter=max_iter, precision=precision)
+        dom.set_field(0, v0)
+        failed = False
+        try:
+            for c in calls:
+                dom.step(c)
+        except gpu._capi.CgError:
+            failed = True
+        return failed, dom
+
+    enough = next(m for m in range(1, 60) if not run(m, [5])[0])
+    out = []
+    for calls in ([10], [1] * 10):
+        failed, dom = run(enough, calls)
+        assert failed and dom.time[1] == 5
+        out.append((dom.time, dom.Vm, dom.Iion, dom.ionic.states(1)))
+    _say("  max_iter", enough, "Iion", np.min(out[0][2]), np.max(out[0][2]))
+    for one, single in zip(*out):
+        np.testing.assert_array_equal(one, single)
