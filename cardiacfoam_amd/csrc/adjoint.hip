@@ -595,7 +595,7 @@ struct Adjoint {
     std::vector<double> h_part;
     int* fail = nullptr;        // a Chebyshev solve missed its tolerance
     double rho = 1.0;           // of the last forward's M
-    bool cg_only = false;       // after such a miss
+    bool cg_only = false;       // the pass of a forward run, or of its gradient, after such a miss
     int last_steps = 0;
     std::vector<double> t0;     // start time of every step of the last forward
     hipStream_t stream;
@@ -850,9 +850,10 @@ static bool adj_missed(Adjoint* A, bool* missed)
     return true;
 }
 
-int adjoint_forward(Adjoint* A, const double* kappa, const double* theta, const int* theta_index,
-                    int n_theta, int n_steps, const std::vector<double>& t0, double* probes,
-                    size_t store_budget, std::string* err)
+static int forward_pass(Adjoint* A, const double* kappa, const double* theta,
+                        const int* theta_index, int n_theta, int n_steps,
+                        const std::vector<double>& t0, double* probes, size_t store_budget,
+                        bool* missed, std::string* err)
 {
     const int64_t n = A->n;
     const unsigned nb = blocks_of(n);
@@ -911,16 +912,11 @@ int adjoint_forward(Adjoint* A, const double* kappa, const double* theta, const 
         if (int rc = adj_step(A, G, t0[st], in, outp, probes + (size_t)st * A->n_probes, err))
             return rc;
     }
-    bool missed;
-    if (!adj_missed(A, &missed)) {
+    if (!adj_missed(A, missed)) {
         *err = "adjoint forward: read-back failed";
         return 4;
     }
-    if (missed) {   // again with the conjugate gradients
-        A->cg_only = true;
-        return adjoint_forward(A, kappa, theta, theta_index, n_theta, n_steps, t0, probes,
-                               store_budget, err);
-    }
+    if (*missed) return 0;
     A->last_steps = n_steps;
     A->t0 = t0;
     const hipError_t e = hipStreamSynchronize(A->stream);
@@ -930,6 +926,24 @@ int adjoint_forward(Adjoint* A, const double* kappa, const double* theta, const 
         return 4;
     }
     return 0;
+}
+
+int adjoint_forward(Adjoint* A, const double* kappa, const double* theta, const int* theta_index,
+                    int n_theta, int n_steps, const std::vector<double>& t0, double* probes,
+                    size_t store_budget, std::string* err)
+{
+    // each run tries Chebyshev's iteration anew: a miss (currents that are not finite, say)
+    // tells nothing about the next kappa and theta
+    A->cg_only = false;
+    bool missed = false;
+    int rc = forward_pass(A, kappa, theta, theta_index, n_theta, n_steps, t0, probes,
+                          store_budget, &missed, err);
+    if (rc == 0 && missed) {   // again with the conjugate gradients
+        A->cg_only = true;
+        rc = forward_pass(A, kappa, theta, theta_index, n_theta, n_steps, t0, probes,
+                          store_budget, &missed, err);
+    }
+    return rc;
 }
 
 int adjoint_backward(Adjoint* A, const double* dprobes, double* dkappa, double* dtheta,
@@ -1001,9 +1015,11 @@ int adjoint_backward(Adjoint* A, const double* dprobes, double* dkappa, double* 
         *err = "adjoint backward: read-back failed";
         return 4;
     }
-    if (missed) {   // again with the conjugate gradients
+    if (missed) {   // again with the conjugate gradients (this pass only)
         A->cg_only = true;
-        return adjoint_backward(A, dprobes, dkappa, dtheta, err);
+        const int rc = adjoint_backward(A, dprobes, dkappa, dtheta, err);
+        A->cg_only = false;
+        return rc;
     }
     std::vector<double> gt(2 * AG);
     hipError_t e = hipMemcpyAsync(gt.data(), A->gtheta, 8 * 2 * AG, hipMemcpyDeviceToHost,
