@@ -309,9 +309,8 @@ void k_cells_protocol(T* __restrict__ st, KParams<T> P, const T* __restrict__ gs
 // results.  The last wave also runs the beat detector, one step behind.
 // Measured (600 steps, FP64, 2048 cells of each model at once): ORd 11.2 -> 5.1 ms, TNNP
 // 7.2 -> 3.2 ms.
-// Up to SPLIT_N cells, one block per CU; beyond that the waves would share SIMDs that one
-// cell per lane fills by itself.
-constexpr int SPLIT_N = 16384;
+// Up to SPLIT_N cells (cg_internal.hpp), one block per CU; beyond that the waves would share
+// SIMDs that one cell per lane fills by itself.
 template <class M> struct SplitRoles {
     static constexpr bool any = false;
 };
@@ -469,7 +468,7 @@ template <class T, bool ADAPTIVE> struct BatchLaunch {
             return go<M, 64, 0, 1>(tissue, states, P, gscale, a, s);
         } else {
             if constexpr (SplitRoles<M>::any) {
-                if (v == 0 && a.n <= SPLIT_N) {
+                if (v == BATCH_SPLIT || (v == BATCH_BY_SIZE && a.n <= SPLIT_N)) {
                     hipLaunchKernelGGL((k_cells_split<M, T>), dim3((unsigned)((a.n + 63) / 64)),
                                        dim3(256), 0, s, (T*)states, kparams<M, T>(P, a.dt),
                                        (const T*)gscale, tissue, a);
@@ -477,6 +476,7 @@ template <class T, bool ADAPTIVE> struct BatchLaunch {
                 }
             }
             switch (v) {
+            case BATCH_BY_SIZE:
             case 0: return go<M, 256, 0>(tissue, states, P, gscale, a, s);
             case 1: return go<M, 64, 0>(tissue, states, P, gscale, a, s);
             case 2: return go<M, 256, 2>(tissue, states, P, gscale, a, s);

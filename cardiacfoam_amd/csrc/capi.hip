@@ -230,7 +230,7 @@ struct cg_ionic {
     int64_t* d_order = nullptr;       // lane -> cell, longest runs first
     int64_t max_len = 0;
     bool lens_set = false;
-    int variant = 0;                  // kernel shape chosen by cg_batch_autotune
+    int variant = cg::BATCH_BY_SIZE;  // kernel shape chosen by cg_batch_autotune
     // beat detection
     int max_beats = 0;
     double beat_thr = 0.0, beat_base_s = 0.0, beat_peak_s = 0.0;  // V/s, s, s
@@ -906,6 +906,7 @@ int cg_batch_autotune(cg_ionic* const* hs, int nh, double dt_s, int trial_steps,
         int best_v = 0;
         char line[160];
         for (int v = 0; v < cg::BATCH_VARIANTS && err == hipSuccess; ++v) {
+            if (!cg::batch_variant_runs(v, h->model, h->n)) continue;
             h->variant = v;
             err = batch_launch(h, dtm, 0, trial_steps, h->stream);  // warm-up
             if (err == hipSuccess) err = hipEventRecord(e0, h->stream);

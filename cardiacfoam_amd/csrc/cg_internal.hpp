@@ -172,7 +172,14 @@ CG_DECLARE_BATCH_ENTRY(fp64)
 CG_DECLARE_BATCH_ENTRY(fp32)
 CG_DECLARE_BATCH_ENTRY(fp64_ode)
 CG_DECLARE_BATCH_ENTRY(fp32_ode)
-constexpr int BATCH_VARIANTS = 6;
+// variants: BATCH_BY_SIZE (a handle not tuned), one cell per lane in one of six shapes, and a
+// cell's step on four waves (TNNP and ORd, the models with SplitRoles) up to SPLIT_N cells
+constexpr int BATCH_BY_SIZE = -1, BATCH_SPLIT = 6, BATCH_VARIANTS = 7;
+constexpr int SPLIT_N = 16384;
+inline bool batch_variant_runs(int v, int model, int64_t n)
+{
+    return v != BATCH_SPLIT || ((model == MODEL_TNNP || model == MODEL_ORD) && n <= SPLIT_N);
+}
 const char* batch_variant_name(int v);
 
 // precision dispatch: prec 0 = fp64, 1 = fp32

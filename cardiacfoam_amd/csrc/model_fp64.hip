@@ -120,7 +120,8 @@ const char* batch_variant_name(int v)
     static const char* names[BATCH_VARIANTS] = {"256 threads", "64 threads",
                                                 "256 threads, >=2 waves/SIMD",
                                                 "64 threads, >=2 waves/SIMD",
-                                                "256 threads, >=3 waves/SIMD", "128 threads"};
+                                                "256 threads, >=3 waves/SIMD", "128 threads",
+                                                "four waves per 64 cells"};
     return v >= 0 && v < BATCH_VARIANTS ? names[v] : "?";
 }
 } // namespace cg

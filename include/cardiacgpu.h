@@ -187,8 +187,8 @@ int cg_ionic_enable_beats(cg_ionic* h, int max_beats, double dvdt_threshold, dou
  * all handles captured in one hipGraph (handles on their own streams run concurrently).
  * Synchronous. */
 int cg_batch_run(cg_ionic* const* handles, int n_handles, double dt_s, int chunk);
-/* Times each kernel shape (threads per block x register budget) on trial_steps steps of
- * every handle, restores the states, keeps the fastest shape per handle; a text report
+/* Times each kernel shape (threads per block x register budget; for small TNNP and ORd
+ * batches also four waves per 64 cells) on trial_steps steps of every handle, restores the states, keeps the fastest shape per handle; a text report
  * goes to report (may be NULL). */
 int cg_batch_autotune(cg_ionic* const* handles, int n_handles, double dt_s, int trial_steps,
                       char* report, size_t report_len);

@@ -156,6 +156,25 @@ def test_batch_autotune_keeps_results(gpu, orc):
     np.testing.assert_allclose(r_t[ok], r_d[ok], rtol=1e-12, atol=0)
 
 
+@pytest.mark.parametrize("name,n,shapes", [("TNNP_epi", 65, 7), ("ORd", 16384, 7),
+                                           ("TNNP_epi", 16385, 6), ("CRN", 64, 6)])
+def test_batch_autotune_names_every_kernel(gpu, orc, name, n, shapes):
+    """Each kernel the autotuner times goes by its own name: the six shapes of one cell per
+    lane, and the four-wave kernel where a batch of that model and size takes it."""
+    _say("batch autotune names", name, n)
+    _, _, key, word, amp = MODELS[name]
+    ion = gpu.IonicModel(key, word, n, solve_vm=True)
+    one = np.ones(n)
+    ion.set_protocol_arrays(5.0 * one, 300.0 * one, one, amp * one, 1, 300.0, 1)
+    ion.set_run_lengths(np.full(n, 40))
+    rep = gpu.batch_autotune([ion], DT_MS * 1e-3, trial_steps=20)
+    _say(rep)
+    timed = [line.split(": ")[1].rsplit(" ", 2)[0] for line in rep.splitlines()
+             if "variant" in line]
+    assert len(timed) == len(set(timed)) == shapes
+    assert ("four waves per 64 cells" in timed) == (shapes == 7)
+
+
 def test_batch_mixed_crossing_zero_mv(gpu, orc):
     """Regression: a TNNP cell whose FP32 Vm passes within 1e-7 mV of 0 mV (seed 20240601,
     cell 340 of the 1,048,576-cell batch) used to hit exp(2 V F/RT) - 1 == 0 in the ICaL
