@@ -5,8 +5,12 @@ linked next to this file.  Run as ``python -m cardiacfoam_amd.build``.
 """
 import concurrent.futures as cf
 import os
+import shutil
 import subprocess
 import sys
+import tempfile
+
+from .listing import masked_reads
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -34,15 +38,39 @@ FAST_F32 = [
 # FP64 Rush-Larsen kernels: instruction selection ordered for register pressure.  With the
 # default source order ORd's tissue kernel spills 167 registers per lane, with this one 39.
 LOW_PRESSURE = ["-mllvm", "-pre-RA-sched=list-burr"]
-EXTRA = {"model_fp64.hip": LOW_PRESSURE, "model_fp32.hip": FAST_F32, "model_fp32_ode.hip": FAST_F32}
+# With many scalar spills this compiler can put a vector register's copy ahead of a restored
+# execution mask (listing.py).  Either of these leaves no such copy in the FP64 model kernels:
+# scalar registers allocated without live-range splitting, or loop-invariant values not moved
+# out of loops (fewer live registers).  The adaptive unit takes the second: under the first
+# one state of Gaur's RKF45 cell kernel is wrong, for a cause that the listing does not show.
+SAFE_SPILLS = ["-mllvm", "-sgpr-regalloc=basic"]
+NO_HOISTS = ["-mllvm", "-disable-machine-licm"]
+EXTRA = {"model_fp64.hip": LOW_PRESSURE + SAFE_SPILLS, "model_fp64_ode.hip": NO_HOISTS,
+         "model_fp32.hip": FAST_F32, "model_fp32_ode.hip": FAST_F32}
 
 
 def _compile(src):
     obj = os.path.join(BUILD, src.replace(".hip", ".o"))
-    cmd = [HIPCC, *FLAGS, *EXTRA.get(src, []), "-c", os.path.join(CSRC, src), "-o", obj]
-    r = subprocess.run(cmd, capture_output=True, text=True)
-    if r.returncode != 0:
-        raise RuntimeError("hipcc failed for %s:\n%s\n%s" % (src, " ".join(cmd), r.stderr))
+    # in a folder of its own, with the intermediate files: the device listing among them is
+    # looked over before it goes
+    tmp = tempfile.mkdtemp(dir=BUILD)
+    try:
+        cmd = [HIPCC, *FLAGS, *EXTRA.get(src, []), "--save-temps=obj", "-c",
+               os.path.join(CSRC, src), "-o", os.path.join(tmp, os.path.basename(obj))]
+        r = subprocess.run(cmd, capture_output=True, text=True)
+        if r.returncode != 0:
+            raise RuntimeError("hipcc failed for %s:\n%s\n%s" % (src, " ".join(cmd), r.stderr))
+        listings = [f for f in os.listdir(tmp) if f.endswith(".s") and "amdgcn" in f]
+        if not listings:
+            raise RuntimeError("no device listing of %s" % src)
+        for f in listings:
+            bad = masked_reads(os.path.join(tmp, f))
+            if bad:
+                raise RuntimeError("%s: registers copied under the wrong lanes in %s" %
+                                   (src, ", ".join("%s %s" % (k, v[:3]) for k, v in bad.items())))
+        os.replace(os.path.join(tmp, os.path.basename(obj)), obj)
+    finally:
+        shutil.rmtree(tmp, ignore_errors=True)
     return obj
 
 

@@ -289,3 +289,36 @@ def test_split_batch_equals_one_cell_per_lane(gpu, orc, name, precision, n):
     np.testing.assert_array_equal(c0, c1)
     np.testing.assert_array_equal(np.isnan(r0), np.isnan(r1))
     np.testing.assert_allclose(np.nan_to_num(r0), np.nan_to_num(r1), rtol=tol, atol=1e-9)
+
+
+@pytest.mark.parametrize("name", ["ORd", "TNNP_epi"])
+def test_split_batch_after_other_kernels(gpu, orc, name):
+    """The four-wave kernel on every compute unit (16384 cells) after kernels that leave their
+    values in all registers: the same states, bit for bit, after each, and those of one cell
+    per lane (a batch of 16385) to 1e-12."""
+    _say("split batch after others", name)
+    _, _, key, word, amp = MODELS[name]
+    big, steps = 16385, 60
+    rng = np.random.default_rng(4)
+    arrays = (rng.uniform(0.0, 0.2, big), 300.0 * np.ones(big), np.ones(big),
+              amp * rng.uniform(1.0, 1.1, big))
+    scale = rng.uniform(0.8, 1.2, (4, big))
+
+    def run(n, key, word, prec="fp64"):
+        ion = gpu.IonicModel(key, word, n, solve_vm=True, precision=prec)
+        ion.set_protocol_arrays(*(a[:n] for a in arrays), 1, 300.0, 1)
+        ion.set_run_lengths(np.full(n, steps))
+        ion.set_conductance_scale(scale[:, :n])
+        gpu.batch_run([ion], DT_MS * 1e-3)
+        return ion.states()
+
+    want = run(big, key, word)[:, :16384]
+    others = [("ToRORd_dynCl", "endocardialCells", "fp64"), ("Grandi", "myocyte", "mixed"),
+              ("Stewart", "myocyte", "fp64"), ("ORd", "myocyte", "mixed")]
+    first = None
+    for o in others:
+        run(16384, *o)
+        got = run(16384, key, word)
+        np.testing.assert_allclose(got, want, rtol=1e-12, atol=1e-15)
+        first = got if first is None else first
+        np.testing.assert_array_equal(got, first)
