@@ -85,7 +85,8 @@ CG_DEV void beat_finish(Beat& b, const BatchArgs& a, int64_t cell, int& nb)
 
 // RL: the Rush-Larsen kernels' detector keeps its ring position and divides without scaling.
 // The adaptive kernels keep the remainder and the plain division: with the new ones a FP64
-// RKF45 batch test ran past its time limit, for a cause not found.
+// RKF45 batch test (TNNP) ran past its time limit; the cause is not shown, so that test is
+// skipped and these kernels keep the former detector.
 template <class T, bool RL> struct Detector {
     const BatchArgs& a;
     int64_t lane, cell;
@@ -309,8 +310,14 @@ void k_cells_protocol(T* __restrict__ st, KParams<T> P, const T* __restrict__ gs
 // results.  The last wave also runs the beat detector, one step behind.
 // Measured (600 steps, FP64, 2048 cells of each model at once): ORd 11.2 -> 5.1 ms, TNNP
 // 7.2 -> 3.2 ms.
-// Up to SPLIT_N cells (cg_internal.hpp), one block per CU; beyond that the waves would share
-// SIMDs that one cell per lane fills by itself.
+// Up to SPLIT_N cells (cg_internal.hpp), one block per CU; beyond that the blocks share CUs
+// and the gain shrinks, for FP64 ORd to nothing.  400 steps in ms, four waves against one cell
+// per lane in 256 threads:
+//    cells    TNNP FP64    TNNP mixed   ORd FP64     ORd mixed
+//   <=16384   1.12  2.77   0.42  0.87   2.46  5.08   0.94  1.50
+//    32768    1.67  2.86   0.54  0.89   4.87  5.12   1.04  1.52
+//    49152    2.44  2.91   0.84  0.90   7.29  5.23   1.85  1.55
+// One line for both models and types: where all four still gain by 1.6 times or more.
 template <class M> struct SplitRoles {
     static constexpr bool any = false;
 };

@@ -232,7 +232,7 @@ __global__ __launch_bounds__(RBS) void k_u(EllView E, double* __restrict__ psi,
 //   FIRST: out = x + r/diag, partials |r| and the normalisation terms;
 //   LAST: the same step, partial |r| of the iterate it starts from;
 //   else: out = xm + omega (x - xm + r/diag), out may be xm.
-// 148k cells: 4.4 us a step where an iteration of k_s and k_u takes 9.8 us.
+// 148k cells: 4.7 us a step where an iteration of k_s and k_u takes 9.8 us.
 template <bool FIRST, bool LAST>
 __global__ __launch_bounds__(RBS) void k_lcheb(EllView E, double omega,
                                                const double* __restrict__ x, const double* xm,

@@ -357,8 +357,10 @@ __global__ __launch_bounds__(MBS) void k_explicit_hex(
     };
     // Models of up to four states: the diffusion part before the model's arithmetic, so that
     // one wait covers the states' and the stencil's loads (a step of a small mesh is the
-    // latency of its chain).  Larger models: after it; its registers held across the model
-    // cost waves, which hide the loads.
+    // latency of its chain): 200 BuenoOrovio steps of 147k cells 1.60 ms, with the loads after
+    // the model 1.65 ms; at 3k cells no difference beyond the runs' own.  Larger models keep
+    // it after the model, where its registers are not held across the model's (not measured
+    // the other way round).
     constexpr bool early = M::NS <= 4;
     if constexpr (early) diffusion();
     const T v = model_v<M, T>(vn);
@@ -388,7 +390,8 @@ __global__ __launch_bounds__(MBS) void k_explicit_hex(
 // waves per SIMD the register allocation of k_ionic_rhs aims at (1: the compiler's
 // choice).  FP64 ORd: 2, at 256 VGPRs with 152 B/lane of spills where one wave takes 256 +
 // 62 AGPRs; with the spills of an earlier build (296 B) it was 4.6 % faster per implicit
-// 2.1M-cell FP64 step.  Grandi (256 + 4 AGPRs at one wave) likewise.
+// 2.1M-cell FP64 step.  Grandi (256 + 4 AGPRs at one wave): 20 implicit FP64 steps of 1M
+// cells 10.3 ms, with one wave 12.1 ms.
 template <class M, class T> constexpr int rhs_waves()
 {
     if constexpr ((std::is_same_v<M, ORd> || std::is_same_v<M, Grandi>) && sizeof(T) == 8) return 2;

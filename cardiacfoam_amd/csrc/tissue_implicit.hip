@@ -264,7 +264,8 @@ CG_DEV T apply_row_diag(const HexOp<T>& A, const Layers<T>& L, const LD& x, int6
            (fyp * (xc - T(x(b.yp))) + fym * (xc - T(x(b.ym)))) +
            (fzp * (xc - T(x(b.zp))) + fzm * (xc - T(x(b.zm))));
 }
-// r / d with the reciprocal's own accuracy (a preconditioner)
+// r / d; FP32 by v_rcp_f32 (1 ulp): the preconditioner shapes the iterates, not the equation
+// that the FP64 residual measures
 CG_DEV float jacobi(float r, float d) { return r * __builtin_amdgcn_rcpf(d); }
 CG_DEV double jacobi(double r, double d) { return div_f64(r, d); }
 template <class T> CG_DEV V4<T> jacobi4(const V4<T>& r, const V4<T>& d)

@@ -52,7 +52,7 @@ def test_batch_adaptive_fp64_vs_oracle(gpu, orc, name, solver):
     integrator to 10 (relTol |y| + absTol); one beat per cell."""
     if (name, solver) == ("TNNP_epi", "RKF45"):
         pytest.skip("ran past its 120 s limit with another beat detector in the kernel; the "
-                    "detector is taken out, not yet run again")
+                    "cause is not shown, so it is not run again")
     _say("batch adaptive fp64", name, solver)
     m, tis = MODELS[name][0], MODELS[name][1]
     n = 3
