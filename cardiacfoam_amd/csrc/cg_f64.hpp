@@ -5,29 +5,17 @@
 // a quarter of the rate, four refinements, quotient, remainder, scaled correction, special
 // cases) and the wait states between them; ORd has 273 divisions in a cell step, 40 % of
 // its instructions.  Written out here without the scalings:
-//   by a constant c      q = a RN(1/c); q + (a - c q) RN(1/c); special cases   (4 or 5)
+//   by a constant c      q = a RN(1/c); q + (a - c q) RN(1/c); special cases   (4)
 //   by a power of two    a (1/c)                                               (1)
-//   1/b                  reciprocal, two refinements, special cases            (7)
-//   a/b                  reciprocal, one refinement, quotient and its
-//                        remainder's correction, special cases                 (8)
-// Error: the hardware's reciprocal is within 2^-24 (2^29 ulp), one refinement brings it
-// to 2^-48, two to rounding.  q is then within 2^-48 of a/b, its remainder is formed in one
-// fma and correct to 2^-53, and the correction (the remainder times the reciprocal) to
-// 2^-48: a relative 2^-96 before the last rounding, so the quotient is within 0.5 + 2^-42 ulp,
-// the correctly rounded one unless a/b lies that close to the middle of two doubles (the
-// order of operations is that of Markstein, IBM J. Res. Dev. 34, 1990, whose theorem asks
-// for a rounded reciprocal).  Below 2^-969 the remainder rounds as a subnormal does.
-// Infinite, zero and NaN operands give IEEE results through v_div_fixup.  What the missing
-// scalings leave are intermediate infinities: a quotient that overflows, and a divisor below
-// 2^-1024, whose reciprocal does; both end as a NaN, which the maximum with -infinity takes
-// away: the quotient is infinite, with IEEE's sign.  (A divisor below 2^-1024 with a finite
-// quotient, for a numerator below 1, gives an infinite one too: a gate's dt/tau, Grandi's and
-// ToRORd's at 1.39 V, where exp(-dt/tau) is 0 either way.)  By a constant of at least 1 no
-// quotient overflows.
-// Measured: 30 implicit FP64 ORd steps of 2.1M cells 34.4 -> 29.3 ms (ionic kernel 732 -> 592
-// us), 200 explicit BuenoOrovio steps of 147k cells 2.10 -> 1.70 ms; the maximum costs 2 to 3 %
-// of the ORd and TNNP kernels (576 us with it, 557 before).  In 6e8 random quotients (a/b, 1/b,
-// by 3, 0.7 and 26.7137; exponents to +-480) none differed from the compiler's division.
+//   1/b                  reciprocal, two refinements, special cases            (6)
+//   a/b                  reciprocal, one refinement, quotient and its exact
+//                        remainder's correction, special cases                 (7)
+// The remainder is exact in one fma, so the quotient is the correctly rounded one as the
+// full expansion's (Markstein, IBM J. Res. Dev. 34, 1990), except where the scalings
+// matter: a divisor outside 2^+-1021 or a quotient that overflows or falls below 2^-969.
+// Infinite, zero and NaN operands give IEEE results through v_div_fixup.
+// Measured: 30 implicit FP64 ORd steps of 2.1M cells 34.4 -> 29.3 ms (ionic kernel 732 ->
+// 592 us), 200 explicit BuenoOrovio steps of 147k cells 2.10 -> 1.70 ms.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <cstdint>
@@ -40,11 +28,6 @@ __host__ __device__ constexpr bool pow2_double(double b)
     return (__builtin_bit_cast(uint64_t, b) & 0xfffffffffffffull) == 0;
 }
 
-__device__ __forceinline__ double div_special(double q, double b, double a)
-{
-    return __builtin_amdgcn_div_fixup(__builtin_fmax(q, -__builtin_inf()), b, a);
-}
-
 __device__ __forceinline__ double div_f64(double a, double b)
 {
     // known after inlining: a constant divisor of ordinary size
@@ -53,15 +36,14 @@ __device__ __forceinline__ double div_f64(double a, double b)
         if (pow2_double(b)) return a * rb;
         const double q = a * rb;
         const double r = __builtin_fma(-b, q, a);
-        const double c = __builtin_fma(r, rb, q);
-        return __builtin_fabs(b) >= 1.0 ? __builtin_amdgcn_div_fixup(c, b, a) : div_special(c, b, a);
+        return __builtin_amdgcn_div_fixup(__builtin_fma(r, rb, q), b, a);
     }
     double r = __builtin_amdgcn_rcp(b);
     r = __builtin_fma(__builtin_fma(-b, r, 1.0), r, r);
     if (__builtin_constant_p(a) && a == 1.0)
-        return div_special(__builtin_fma(__builtin_fma(-b, r, 1.0), r, r), b, a);
+        return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-b, r, 1.0), r, r), b, a);
     const double q = a * r;
-    return div_special(__builtin_fma(__builtin_fma(-b, q, a), r, q), b, a);
+    return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-b, q, a), r, q), b, a);
 }
 
 struct F64 {
