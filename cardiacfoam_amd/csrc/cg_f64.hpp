@@ -10,10 +10,18 @@
 //   1/b                  reciprocal, two refinements, special cases            (6)
 //   a/b                  reciprocal, one refinement, quotient and its exact
 //                        remainder's correction, special cases                 (7)
-// The remainder is exact in one fma, so the quotient is the correctly rounded one as the
-// full expansion's (Markstein, IBM J. Res. Dev. 34, 1990), except where the scalings
-// matter: a divisor outside 2^+-1021 or a quotient that overflows or falls below 2^-969.
-// Infinite, zero and NaN operands give IEEE results through v_div_fixup.
+// Error: the hardware's reciprocal is within 2^-24 (2^29 ulp), one refinement brings it
+// to 2^-48, two to rounding.  q is then within 2^-48 of a/b, its remainder is formed in one
+// fma and correct to 2^-53, and the correction (the remainder times the reciprocal) to
+// 2^-48: a relative 2^-96 before the last rounding, so the quotient is within 0.5 + 2^-42 ulp,
+// the correctly rounded one unless a/b lies that close to the middle of two doubles (the
+// order of operations is that of Markstein, IBM J. Res. Dev. 34, 1990, whose theorem asks
+// for a rounded reciprocal).  Below 2^-969 the remainder rounds as a subnormal does.
+// Infinite, zero and NaN operands and overflowing quotients give IEEE results through
+// v_div_fixup (measured).  A divisor below 2^-1024 with a finite quotient gives an infinite
+// one: a gate's dt/tau, Grandi's and ToRORd's at 1.39 V, where exp(-dt/tau) is 0 either way.
+// In 6e8 random quotients (a/b, 1/b, by 3, 0.7 and 26.7137; exponents to +-480) none differed
+// from the compiler's division.
 // Measured: 30 implicit FP64 ORd steps of 2.1M cells 34.4 -> 29.3 ms (ionic kernel 732 ->
 // 592 us), 200 explicit BuenoOrovio steps of 147k cells 2.10 -> 1.70 ms.
 #pragma once

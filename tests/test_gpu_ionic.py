@@ -135,3 +135,33 @@ def test_states_round_trip_in_pieces(gpu, orc, precision, n):
         np.testing.assert_array_equal(got, want)
     else:
         assert np.all(np.abs(got - want) <= 6e-8 * np.abs(want) + 1e-12)
+
+
+@pytest.mark.parametrize("name,lo,hi", [("TNNP_epi", -3.7, -3.5), ("STW", -3.7, -3.5),
+                                        ("GRD", -1.5, -1.3), ("GRD", 1.3, 1.5),
+                                        ("TOR_M", -1.5, -1.3), ("TOR_M", 1.3, 1.5)])
+def test_gates_whose_time_constant_is_subnormal(gpu, orc, name, lo, hi):
+    """Potentials (V) around the one at which an exponential overflows and a gate's time
+    constant falls below 2^-1022 and then to 0: dt / tau is finite, then infinite, never NaN,
+    and the gate lands on its target, as the oracle's.  1e-10 relative (an exponential of 700
+    carries 700 roundings of its argument: 1e-13); a concentration that a current of 1e30
+    drives out of any range is only compared as finite or not."""
+    _say("subnormal time constants", name, lo, hi)
+    m, tis, key, word, _ = MODELS[name]
+    n, dt = 4001, 1e-5
+    c, states, _ = physiological_states(orc, name, n, seed=7)
+    V = np.linspace(lo, hi, n)
+    ion = gpu.IonicModel(key, word, n, solve_vm=False)
+    ion.set_states(states)
+    Im = np.zeros(n)
+    ion.solveODE(0.0, dt, V, Im)
+    ref = states.copy()
+    Im_ref = orc.ionic_tissue_step(m, tis, c, ref, 0.0, dt, V, integrator=0)
+    got = ion.states()
+    _say("  finite: oracle %.4f, device %.4f" % (np.isfinite(ref[1:]).mean(),
+                                                 np.isfinite(got[1:]).mean()))
+    np.testing.assert_array_equal(np.isfinite(got[1:]), np.isfinite(ref[1:]))
+    ok = np.abs(ref[1:]) < 1e3
+    assert ok.mean() > 0.9
+    np.testing.assert_allclose(got[1:][ok], ref[1:][ok], rtol=1e-10, atol=1e-14)
+    np.testing.assert_array_equal(np.isfinite(Im), np.isfinite(Im_ref))
